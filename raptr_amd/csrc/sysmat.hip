@@ -124,7 +124,12 @@ constexpr int kCountStride = 16;  // counters are 128 bytes apart
 
 struct BuildArgs {
   Geom G;
-  FastDiv div_yz, div_z, div_x, div_pl;
+  FastDiv div_yz, div_z;
+  FastDiv div_c[4];     // channels per angle, id0z, id0y, id1z
+  // k_sm_rays: 1 / pitch, farthest plane from 0, half a voxel's diagonal
+  float inv_d[3], ext[3];
+  float near2;       // squared end offset up to which no voxel can fail the cull
+  bool plain_planes; // plane positions are 0 or of moderate size
   int rpb;          // rays per mask bit (k_sm_rays)
   const int* list;  // nullptr: channel = list index (all channels)
   int first;        // first list entry of this launch
@@ -133,6 +138,7 @@ struct BuildArgs {
   uint32_t seed;
   int raygen;
   int keep_zeros;   // store zero-valued candidates too (RAPTR_SM_KEEP_ZEROS)
+  int by_candidate; // k_sm_build whatever the rays
   int pl;           // planes per ray (nx+1 + ny+1 + nz+1)
   // outputs
   int* row_nnz;     // [rows]
@@ -221,11 +227,15 @@ __device__ inline float sample_element(const Geom& G, uint32_t seed, int nrays, 
   return a / float(nrays);
 }
 
+// staging area of a row (hashed: row lengths repeat with the pixel index)
+__device__ inline int staging_area(const BuildArgs& A, int rl) {
+  return A.areas == kAreas ? int((uint32_t(rl) * 0x9E3779B1u) >> 26) : 0;
+}
+
 // Staging offset of a piece of n entries of row rl (`within`: entries of the
 // row before it), entered in the piece table; -1 (and a flag) if full.
 __device__ inline long long reserve_piece(const BuildArgs& A, int rl, int within, int n) {
-  // (hashed: row lengths repeat with the pixel index)
-  const int area = A.areas == kAreas ? int((uint32_t(rl) * 0x9E3779B1u) >> 26) : 0;
+  const int area = staging_area(A, rl);
   const long long off = (long long)atomicAdd(&A.st_count[area * kCountStride],
                                              (unsigned long long)n);
   if (off + n > A.st_cap) {
@@ -498,7 +508,7 @@ __global__ __launch_bounds__(kSmBlock) void k_sm_build(BuildArgs A) {
 // k_sm_build tests every culled voxel against every ray, and 95 % of its
 // candidates turn out to be zero.  Here each ray marks the voxels that it can
 // cross, so only those are sampled, by the rays that marked them:
-//   1. the channel's rays and plane tables in LDS, as in k_sm_build;
+//   1. the channel's rays and their plane tables in LDS, as in k_sm_build;
 //   2. the grid is cut into slabs along x or z, whichever the line runs along;
 //      per (ray, slab) the cells that the ray can cross there on the two
 //      other axes form two ranges, widened by more than their rounding error.
@@ -510,14 +520,19 @@ __global__ __launch_bounds__(kSmBlock) void k_sm_build(BuildArgs A) {
 //      voxel ANDed; a voxel with bits left is summed over the rays of those
 //      bits in ascending order, with k_sm_build's arithmetic.  A ray that
 //      is not in the mask does not cross the voxel, its term would be +0, so
-//      sums are the same bit for bit; non-zero ones get the cylinder test.
-// More than 32 rays share bits in runs of `rpb` consecutive rays.
-// Bound by VALU and LDS latency: 100,003 rows of the 52^3 / 30-ray geometry
-// (36M entries) take 3.0 ms against 58 ms with k_sm_build.
+//      sums are the same bit for bit.
+// On the 52^3 / 30-ray geometry a row walks 446 voxels, 361 keep bits and 358
+// are non-zero (k_sm_build: 5,900 candidates).  More than 32 rays share bits
+// in runs of `rpb` consecutive rays.
+// Bound by VALU issue (80 % busy) and LDS latency: 1,920 VALU instructions a
+// wave and row, a quarter each in the plane tables and the masks.  Measured,
+// k_sm_build -> masks -> with the voxels in order of their bits, odd table
+// strides, one staging request a row and half the barriers: 100,003 rows of
+// that geometry 58.0 -> 3.25 -> 1.78 ms, 20,011 rows of 96^3 / 20 rays 17.0 ->
+// 0.90 -> 0.66 ms, sensitivity of 147,456 channels (32^3 / 10 rays) 16.9 ->
+// 1.19 -> 0.96 ms.
 constexpr int kMw = 8;              // mask words per slab and axis
-constexpr int kMChunk = 256;        // voxels of a wave's share of a segment
-constexpr int kMWaves = kSmBlock / kWave;
-constexpr int kMRow = kMChunk * kMWaves;  // row buffer: a segment always fits
+constexpr int kMRow = 768;          // voxels of a segment; entries of the row buffer
 
 __device__ inline float min2(float a, float b) {
   float r;
@@ -540,61 +555,76 @@ __device__ inline float max3(float a, float b, float c) {
   return r;
 }
 
-// Cells [c0, c1] of an axis that a ray r0 + a*d can cross for a in [lo, hi]
-// (d == 0: the slab method ignores the axis, so all of them).  The position's
-// rounding error and that of the plane tables stay below 2^-21 of the sizes
-// that enter; the ranges are widened by twice that.
-__device__ inline bool cell_range(int n, float r0, float d, float o, float inv, float ext,
-                                  float lo, float hi, int& c0, int& c1) {
-  if (d == 0.0f) {
-    c0 = 0;
-    c1 = n - 1;
-    return true;
-  }
-  const float a = lo * d, b = hi * d;
-  const float ea = (fabsf(r0) + fabsf(a) + ext) * 9.5367431640625e-7f;
-  const float eb = (fabsf(r0) + fabsf(b) + ext) * 9.5367431640625e-7f;
-  const float ya = (r0 + a) - o, yb = (r0 + b) - o;
-  const float y0 = d > 0.0f ? (ya - ea) * inv : (yb - eb) * inv;
-  const float y1 = d > 0.0f ? (yb + eb) * inv : (ya + ea) * inv;
-  // clamped before the conversion; a NaN (infinite bounds) gives the full range
-  c0 = int(fminf(fmaxf(floorf(y0), 0.0f), float(n)));
-  c1 = int(fmaxf(fminf(floorf(y1), float(n - 1)), -1.0f));
-  return c0 <= c1;
+// Position of a ray on an axis in cells as base + a * slope, and the bound of
+// its rounding error, that of the plane tables included: every term is below
+// 2^-23 of (|r0| + ext) * inv, ext the farthest plane; eps is 32 of them.  A
+// ray that does not cross the axis is not bounded there: eps infinite.
+__device__ inline void axis_line(float r0, float d, float o, float inv, float ext, float* out) {
+  out[0] = d != 0.0f ? (r0 - o) * inv : 0.0f;
+  out[1] = d * inv;
+  out[2] = d != 0.0f ? (fabsf(r0) + ext) * inv * 3.814697265625e-6f : __builtin_inff();
 }
 
-// Wave-private LDS lists: the lanes of one wave run in step and their LDS
-// accesses are issued in program order; the compiler must keep that order.
+// floor to int; out of int range: its nearest end
+__device__ inline int floor_int(float a) {
+  int r;
+  asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(a));
+  return r;
+}
+
+// Cells [c0, c1] that the ray can cross for a in [lo, hi] (finite); empty if
+// c0 > c1.
+__device__ inline void cell_range(const float* line, int n, float lo, float hi, int& c0, int& c1) {
+  const float pa = __builtin_fmaf(lo, line[1], line[0]);
+  const float pb = __builtin_fmaf(hi, line[1], line[0]);
+  c0 = floor_int(min2(pa, pb) - line[2]);
+  c1 = floor_int(max2(pa, pb) + line[2]);
+  c0 = c0 > 0 ? c0 : 0;
+  c1 = c1 < n - 1 ? c1 : n - 1;
+}
+
+// Words that every wave writes alike and reads back: LDS accesses of a wave
+// are issued in program order; the compiler must keep that order.
 __device__ inline void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
 }
 
-template <int MODE, bool ONE>
-__global__ __launch_bounds__(kSmBlock) void k_sm_rays(BuildArgs A) {
+// a is 0 or of magnitude 2^-e .. 2^e
+__host__ __device__ inline bool plain_size(float a, int e) {
+  const float b = a < 0.0f ? -a : a;
+  return b == 0.0f ? e == 60 : b >= 1.0f / float(1ull << e) && b <= float(1ull << e);
+}
+
+template <int MODE, bool ONE, int NW>
+__global__ __launch_bounds__(NW * kWave) void k_sm_rays(BuildArgs A) {
+  constexpr int NT = NW * kWave, CH = kMRow / NW;  // CH: a wave's voxels of a segment
   extern __shared__ float smem[];
-  __shared__ int s_wn[kMWaves];
-  __shared__ int s_scan[kMWaves];
-  __shared__ int s_rect[kSmBlock][4];  // y0, z0, z cells, area prefix of an x index
-  __shared__ double s_red[kMWaves];
+  __shared__ int s_wn[NW], s_kept[NW], s_cull[NW];
+  __shared__ float s_dev[NW];
+  __shared__ int s_pre[kWave], s_wz[kWave];  // of an x index: voxels before it, z cells
+  __shared__ int s_bin[32], s_place[32];     // voxels by number of mask bits
+  __shared__ unsigned short s_ord[kMRow];    // list positions, most bits first
+  __shared__ double s_red[NW];
   __shared__ long long s_off;
   const int nr = A.nrays, pl = A.pl;
   const int nx = A.G.g.n[0], ny = A.G.g.n[1], nz = A.G.g.n[2];
   const int off1 = nx + 1, off2 = nx + 1 + ny + 1;
   const int nsm = nx > nz ? nx : nz;
-  float* rpos = smem;                                      // nr * 8: start, direction
-  float* rlen = rpos + 8 * nr;                             // nr
-  float* alpha = rlen + nr;                                // nr * pl
-  unsigned* my = reinterpret_cast<unsigned*>(alpha + size_t(nr) * pl);  // nsm * kMw
+  // plane table and length of a ray, an odd number of words: the rays of a
+  // wave's lanes then lie in different banks
+  const int stride = (pl + 1) | 1;
+  float* alpha = smem;                                     // nr * stride
+  unsigned* my = reinterpret_cast<unsigned*>(alpha + size_t(nr) * stride);  // nsm * kMw
   unsigned* mt = my + nsm * kMw;                           // nsm * kMw
   int* ylo = reinterpret_cast<int*>(mt + nsm * kMw);       // nx each
   int* yhi = ylo + nx;
   int* zlo = yhi + nx;
   int* zhi = zlo + nx;
-  int* l_vox = zhi + nx;                                   // kMWaves * kMChunk
+  // the rays (16 floats each) until the masks stand, then the wave lists
+  int* l_vox = zhi + nx;                                   // NW * CH
   unsigned* l_bit = reinterpret_cast<unsigned*>(l_vox + kMRow);  // mask, then value
-  int* rb_col = reinterpret_cast<int*>(l_bit + kMRow);     // kMRow (fill)
-  float* rb_val = reinterpret_cast<float*>(rb_col + kMRow);
+  float* rays = reinterpret_cast<float*>(l_vox);
 
   const int t = threadIdx.x, lane = t & (kWave - 1), w = t / kWave;
   const int rl = blockIdx.x;
@@ -608,14 +638,31 @@ __global__ __launch_bounds__(kSmBlock) void k_sm_rays(BuildArgs A) {
     }
     return;
   }
-  int ida, id0z, id0y, id1z, id1y;
-  cnl_split(A.G.s, cnl, ida, id0z, id0y, id1z, id1y);
+  // cnl_split by multiplications (the channel is uniform: scalar unit)
+  uint32_t q = uint32_t(cnl);
+  const int ida = int(fdiv(q, A.div_c[0]));
+  q -= uint32_t(ida) * A.div_c[0].d;
+  const int id0z = int(fdiv(q, A.div_c[1]));
+  q -= uint32_t(id0z) * A.div_c[1].d;
+  const int id0y = int(fdiv(q, A.div_c[2]));
+  q -= uint32_t(id0y) * A.div_c[2].d;
+  const int id1z = int(fdiv(q, A.div_c[3]));
+  const int id1y = int(q - uint32_t(id1z) * A.div_c[3].d);
   const float sn = A.G.sn[ida], cs = A.G.cs[ida];
+  float p0[3], p1[3];
+  trafo(A.G.s, 0, sn, cs, id0z, id0y, 0.5f, 0.5f, 0.5f, p0);
+  trafo(A.G.s, 1, sn, cs, id1z, id1y, 0.5f, 0.5f, 0.5f, p1);
+  // slabs along the axis that the line runs along
+  const bool zs = fabsf(p1[2] - p0[2]) > fabsf(p1[0] - p0[0]);
+  const int ns = zs ? nz : nx, nt = zs ? nx : nz;
+  const int td = zs ? 0 : 2;
   // rays: lane 2k makes the start of ray k, lane 2k + 1 its end (the
   // uniforms of make_ray: three words of the first Philox block, then its
   // fourth and two of the second)
-  for (int q = t; q < ((2 * nr + kWave - 1) & ~(kWave - 1)); q += kSmBlock) {
-    const int r = q >> 1, det = q & 1;
+  float far_end = 0.0f;  // largest squared distance of a ray's end from its pixel centre
+  bool cullw = false;    // a ray that does not follow the line between the heads
+  for (int k = t; k < ((2 * nr + kWave - 1) & ~(kWave - 1)); k += NT) {
+    const int r = k >> 1, det = k & 1;
     float b0 = 0.5f, b1 = 0.5f, b2 = 0.5f;
     if (A.raygen != RAPTR_RAYGEN_REGU) {
       uint32_t o[4];
@@ -625,250 +672,333 @@ __global__ __launch_bounds__(kSmBlock) void k_sm_rays(BuildArgs A) {
       b1 = u01(det ? o[0] : o[1]);
       b2 = u01(det ? o[1] : o[2]);
     }
-    float e[3], d[3];
+    float e[3], d[3], dev = 0.0f;
     trafo(A.G.s, det, sn, cs, det ? id1z : id0z, det ? id1y : id0y, b0, b1, b2, e);
     bool same = true;
-    for (int k = 0; k < 3; ++k) {
-      const float far = __shfl_xor(e[k], 1, kWave);  // lane 2k: the ray's end
-      same = same && e[k] == far;
-      d[k] = far - e[k];
+    for (int j = 0; j < 3; ++j) {
+      const float far = __shfl_xor(e[j], 1, kWave);  // lane 2k: the ray's end
+      same = same && e[j] == far;
+      d[j] = far - e[j];
+      const float off = e[j] - (det ? p1[j] : p0[j]);
+      dev += off * off;
     }
+    if (r < nr) far_end = max2(far_end, dev);
+    cullw = cullw || (r < nr && (d[0] == 0.0f || d[1] == 0.0f || d[2] == 0.0f));
     if (det == 0 && r < nr) {
-      for (int k = 0; k < 3; ++k) {
-        rpos[8 * r + k] = e[k];
-        rpos[8 * r + 4 + k] = d[k];
+      float* ri = rays + 16 * r;
+      for (int j = 0; j < 3; ++j) {
+        ri[j] = e[j];
+        ri[4 + j] = d[j];
       }
-      // a ray without length crosses nothing
-      rpos[8 * r + 3] = same ? 0.0f : 1.0f;
-      rlen[r] = sqrtf(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
+      bool plain = A.plain_planes;
+      for (int j = 0; j < 3; ++j) plain = plain && plain_size(d[j], 40) && plain_size(e[j], 60);
+      ri[3] = same ? 0.0f : plain ? 2.0f : 1.0f;
+      axis_line(e[1], d[1], A.G.g.o[1], A.inv_d[1], A.ext[1], ri + 8);
+      axis_line(zs ? e[0] : e[2], zs ? d[0] : d[2], A.G.g.o[td], A.inv_d[td], A.ext[td],
+                ri + 12);
+      ri[7] = 1.0f / d[2];
+      ri[11] = 1.0f / d[0];
+      ri[15] = 1.0f / d[1];
+      alpha[r * stride + pl] = sqrtf(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
     }
   }
-  for (int k = t; k < 2 * nsm * kMw; k += kSmBlock) my[k] = 0u;
-  for (int k = t; k < nx; k += kSmBlock) {
+  for (int j = kWave / 2; j > 0; j >>= 1) far_end = max2(far_end, __shfl_xor(far_end, j, kWave));
+  if (lane == 0) s_dev[w] = far_end;
+  if (t < 32) s_bin[t] = s_place[t] = 0;
+  for (int k = t; k < 2 * nsm * kMw; k += NT) my[k] = 0u;
+  for (int k = t; k < nx; k += NT) {
     ylo[k] = zlo[k] = 0x7fffffff;
     yhi[k] = zhi[k] = -1;
   }
-  float p0[3], p1[3];
-  trafo(A.G.s, 0, sn, cs, id0z, id0y, 0.5f, 0.5f, 0.5f, p0);
-  trafo(A.G.s, 1, sn, cs, id1z, id1y, 0.5f, 0.5f, 0.5f, p1);
   __syncthreads();
-  // plane tables.  An axis that the ray does not cross is ignored by the slab
-  // method: alternating infinities leave every cell unbounded there.
-  for (int k = t; k < nr * pl; k += kSmBlock) {
-    const int r = int(fdiv(uint32_t(k), A.div_pl)), p = k - r * pl;
+  // plane tables: a lane keeps its plane, a wave takes every NW-th ray
+  for (int p0_ = 0; p0_ < pl; p0_ += kWave) {
+    const int p = p0_ + lane;
     const int dim = p < off1 ? 0 : (p < off2 ? 1 : 2);
     const int idx = p - (dim == 0 ? 0 : (dim == 1 ? off1 : off2));
-    const float* ri = rpos + 8 * r;
-    const float d = ri[4 + dim];
-    float v = ((idx & 1) ? 1.0f : -1.0f) * __builtin_inff();
-    if (d != 0.0f) v = (plane(A.G.g, dim, idx) - ri[dim]) / d;
-    alpha[k] = ri[3] != 0.0f ? v : 0.0f;
+    const int inv = dim == 0 ? 11 : dim == 1 ? 15 : 7;
+    const float pos = plane(A.G.g, dim, idx);
+    if (p < pl)
+      for (int r = w; r < nr; r += NW) {
+        const float* ri = rays + 16 * r;
+        const float a = pos - ri[dim], d = ri[4 + dim];
+        float v;
+        if (__builtin_amdgcn_readfirstlane(__float_as_int(ri[3])) == 0x40000000) {
+          // a / d from the rounded reciprocal: two residual steps give the
+          // correctly rounded quotient (Markstein, IBM J. Res. Dev. 34, 1990)
+          // where neither it nor the residuals leave the normal range
+          const float y = ri[inv];
+          v = a * y;
+          v = __builtin_fmaf(__builtin_fmaf(-v, d, a), y, v);
+          v = __builtin_fmaf(__builtin_fmaf(-v, d, a), y, v);
+        } else {
+          // a ray without length crosses nothing; an axis that the ray does
+          // not cross is ignored by the slab method: alternating infinities
+          // leave every cell unbounded there
+          v = ((idx & 1) ? 1.0f : -1.0f) * __builtin_inff();
+          if (d != 0.0f) v = a / d;
+          if (ri[3] == 0.0f) v = 0.0f;
+        }
+        alpha[r * stride + p] = v;
+      }
   }
   __syncthreads();
-  // masks and rectangles; slabs along the axis that the line runs along
-  const bool zs = fabsf(p1[2] - p0[2]) > fabsf(p1[0] - p0[0]);
-  const int ns = zs ? nz : nx, nt = zs ? nx : nz;
-  const int td = zs ? 0 : 2;
-  const int soff = zs ? off2 : 0;
-  const FastDiv div_s = zs ? A.div_z : A.div_x;
-  const float yo = A.G.g.o[1], to = A.G.g.o[td];
-  const float yi = 1.0f / A.G.g.d[1], ti = 1.0f / A.G.g.d[td];
-  const float ye = fabsf(yo) + float(ny) * A.G.g.d[1];
-  const float te = fabsf(to) + float(nt) * A.G.g.d[td];
-  for (int k = t; k < nr * ns; k += kSmBlock) {
-    const int r = int(fdiv(uint32_t(k), div_s)), sl = k - r * ns;
-    const float* ri = rpos + 8 * r;
-    const float* al = alpha + size_t(r) * pl + soff + sl;
-    const float a0 = al[0], a1 = al[1];
-    const float lo = min2(a0, a1), hi = max2(a0, a1);
-    int y0, y1, t0, t1;
-    if (ri[3] == 0.0f || lo >= hi) continue;
-    if (!cell_range(ny, ri[1], ri[5], yo, yi, ye, lo, hi, y0, y1)) continue;
-    if (!cell_range(nt, ri[td], ri[4 + td], to, ti, te, lo, hi, t0, t1)) continue;
-    const unsigned bit = 1u << (ONE ? r : r / A.rpb);
-    const int cy = y1 - y0 + 1 < kMw ? y1 - y0 + 1 : kMw;
-    const int ct = t1 - t0 + 1 < kMw ? t1 - t0 + 1 : kMw;
-    for (int j = 0; j < cy; ++j) atomicOr(&my[sl * kMw + ((y0 + j) & (kMw - 1))], bit);
-    for (int j = 0; j < ct; ++j) atomicOr(&mt[sl * kMw + ((t0 + j) & (kMw - 1))], bit);
-    const int x0 = zs ? t0 : sl, x1 = zs ? t1 : sl;
-    for (int x = x0; x <= x1; ++x) {
-      atomicMin(&ylo[x], y0);
-      atomicMax(&yhi[x], y1);
-      atomicMin(&zlo[x], zs ? sl : t0);
-      atomicMax(&zhi[x], zs ? sl : t1);
+  // masks, and the window of cells per slab: a lane keeps its slab
+  for (int s0 = 0; s0 < ns; s0 += kWave) {
+    const int sl = s0 + lane;
+    int wy0 = 0x7fffffff, wy1 = -1, wt0 = 0x7fffffff, wt1 = -1;
+    if (sl < ns)
+      for (int r = w; r < nr; r += NW) {
+        const float* ri = rays + 16 * r;
+        const float* al = alpha + r * stride + (zs ? off2 : 0) + sl;
+        const float a0 = al[0], a1 = al[1];
+        // (an uncrossed slab axis leaves infinities)
+        const float lo = max2(min2(a0, a1), -1e30f), hi = min2(max2(a0, a1), 1e30f);
+        int y0, y1, t0, t1;
+        cell_range(ri + 8, ny, lo, hi, y0, y1);
+        cell_range(ri + 12, nt, lo, hi, t0, t1);
+        if (y0 > y1 || t0 > t1 || ri[3] == 0.0f || lo >= hi) continue;
+        cullw = cullw || lo < 0.0f || hi > 1.0f;
+        const unsigned bit = 1u << (ONE ? r : r / A.rpb);
+        wy0 = y0 < wy0 ? y0 : wy0;
+        wy1 = y1 > wy1 ? y1 : wy1;
+        wt0 = t0 < wt0 ? t0 : wt0;
+        wt1 = t1 > wt1 ? t1 : wt1;
+        unsigned* sy = my + sl * kMw;
+        unsigned* st = mt + sl * kMw;
+        // mostly one or two cells; kMw of them reach every word
+        atomicOr(&sy[y0 & (kMw - 1)], bit);
+        atomicOr(&sy[y1 & (kMw - 1)], bit);
+        atomicOr(&st[t0 & (kMw - 1)], bit);
+        atomicOr(&st[t1 & (kMw - 1)], bit);
+        if (y1 - y0 > 1 || t1 - t0 > 1) {
+          y1 = y1 - y0 < kMw ? y1 : y0 + kMw;
+          t1 = t1 - t0 < kMw ? t1 : t0 + kMw;
+          while (++y0 < y1) atomicOr(&sy[y0 & (kMw - 1)], bit);
+          while (++t0 < t1) atomicOr(&st[t0 & (kMw - 1)], bit);
+        }
+      }
+    if (wy1 >= 0) {
+      const int x0 = zs ? wt0 : sl, x1 = zs ? wt1 : sl;
+      for (int x = x0; x <= x1; ++x) {
+        atomicMin(&ylo[x], wy0);
+        atomicMax(&yhi[x], wy1);
+        atomicMin(&zlo[x], zs ? sl : wt0);
+        atomicMax(&zhi[x], zs ? sl : wt1);
+      }
     }
   }
+  if (lane == 0) s_cull[w] = 0;
+  if (cullw) s_cull[w] = 1;
   __syncthreads();
 
-  int rb_n = 0, flushed = 0;  // fill: entries in the row buffer, flushed before
-  int count = 0;              // count: this wave's entries
+  // Between the heads a ray is no farther from the channel's line than the
+  // farther of its ends from its pixel centre, so a voxel that it crosses is
+  // within that and half the voxel's diagonal of the line: mostly less than
+  // the cull's radius for all rays, by more than the test's rounding error,
+  // and no voxel needs the test.  It stays where a ray does not cross an axis
+  // (the slab method then takes voxels off the ray) or is crossed outside.
+  bool cull = false;
+  for (int ww = 0; ww < NW; ++ww) {
+    cull = cull || s_cull[ww];
+    far_end = max2(far_end, s_dev[ww]);
+  }
+  cull = cull || !(far_end < A.near2);
+
+  int row_n = 0;  // fill: entries of the row so far
+  int count = 0;  // count: this thread's entries
   double proj = 0.0;
   const double wt = (MODE == kModeColsum && A.wgt) ? double(A.wgt[li]) : 1.0;
-  auto flush = [&]() {
-    if (t == 0) s_off = reserve_piece(A, rl, flushed, rb_n);
-    __syncthreads();
-    const long long o = s_off;
-    if (o >= 0)
-      for (int k = t; k < rb_n; k += kSmBlock) {
-        A.st_col[o + k] = rb_col[k];
-        A.st_val[o + k] = rb_val[k];
-      }
-    flushed += rb_n;
-    rb_n = 0;
-    __syncthreads();
-  };
-  int* wv = l_vox + w * kMChunk;
-  unsigned* wb = l_bit + w * kMChunk;
+  // fill: room for a voxel of every rectangle in the staging, one request a
+  // row (its answer is waited for when the first entries are written)
+  unsigned long long room = 0;
+  int vox_all = 0;
+  if (MODE == kModeFill) {
+    for (int x = lane; x < nx; x += kWave)
+      if (yhi[x] >= ylo[x]) vox_all += (yhi[x] - ylo[x] + 1) * (zhi[x] - zlo[x] + 1);
+    vox_all = wave_reduce_sum(vox_all);
+    if (t == 0) room = atomicAdd(&A.st_count[staging_area(A, rl) * kCountStride],
+                                 (unsigned long long)vox_all);
+  }
+  int* wv = l_vox + w * CH;
+  unsigned* wb = l_bit + w * CH;
   // items [k0, k1) of the current rectangles, by one wave: voxels with bits
-  // left, listed in order, then sampled; the non-zero ones that pass the cull
-  // stay in the list (fill).  Returns their number.
-  auto wave_items = [&](int k0, int k1, int xb, int xn) -> int {
+  // left, listed in order and counted by their number of bits
+  auto list_items = [&](int k0, int k1, int xb) -> int {
     int n = 0;
     for (int k = k0 + lane; k - lane < k1; k += kWave) {
       unsigned m = 0u;
       int v = 0;
       if (k < k1) {
-        int jl = 0, jh = xn - 1;  // last x index with prefix <= k
-        while (jl < jh) {
-          const int mid = (jl + jh + 1) >> 1;
-          if (s_rect[mid][3] <= k) jl = mid; else jh = mid - 1;
-        }
-        const int q = k - s_rect[jl][3], wz = s_rect[jl][2];
+        int jl = 0;  // last x index with prefix <= k
+#pragma unroll
+        for (int j = kWave / 2; j > 0; j >>= 1)
+          if (s_pre[jl + j] <= k) jl += j;
+        const int ix = xb + jl;
+        const int q = k - s_pre[jl], wz = s_wz[jl];
         int qy = int((float(q) + 0.5f) * __builtin_amdgcn_rcpf(float(wz)));
-        int qz = q - qy * wz;
+        int qz = q - int(__umul24(unsigned(qy), unsigned(wz)));
         if (qz < 0) qz += wz, --qy;
         if (qz >= wz) qz -= wz, ++qy;
-        const int ix = xb + jl, iy = s_rect[jl][0] + qy, iz = s_rect[jl][1] + qz;
+        const int iy = ylo[ix] + qy, iz = zlo[ix] + qz;
         const int sl = zs ? iz : ix, tt = zs ? ix : iz;
         m = my[sl * kMw + (iy & (kMw - 1))] & mt[sl * kMw + (tt & (kMw - 1))];
-        v = (ix * ny + iy) * nz + iz;
+        v = int(__umul24(unsigned(__umul24(unsigned(ix), unsigned(ny)) + iy), unsigned(nz))) + iz;
       }
       const uint64_t b = __ballot(m != 0u);
       if (m) {
         const int pos = n + __popcll(b & lanemask_lt());
         wv[pos] = v;
         wb[pos] = m;
+        atomicAdd(&s_bin[32 - __popc(m)], 1);
       }
       n += __popcll(b);
     }
-    wave_lds_fence();
-    int kept = 0;
-    for (int c = lane; c - lane < n; c += kWave) {
-      float a = 0.0f;
-      int v = 0;
-      if (c < n) {
-        v = wv[c];
-        unsigned m = wb[c];
-        const int ix = int(fdiv(uint32_t(v), A.div_yz));
-        const int rem = v - ix * int(A.div_yz.d);
-        const int iy = int(fdiv(uint32_t(rem), A.div_z));
-        const int iz = rem - iy * nz;
-        const float* ax = alpha + ix;
-        const float* ay = alpha + off1 + iy;
-        const float* az = alpha + off2 + iz;
-        while (m) {
-          const int b = __ffs(int(m)) - 1;
-          m &= m - 1u;
-          const int r0 = ONE ? b : b * A.rpb;
-          const int r1 = ONE ? b + 1 : (r0 + A.rpb < nr ? r0 + A.rpb : nr);
-          for (int r = r0; r < r1; ++r) {
-            const int o = r * pl;
-            const float xa = ax[o], xb_ = ax[o + 1], ya = ay[o], yb = ay[o + 1];
-            const float za = az[o], zb = az[o + 1];
-            const float lo = max3(min2(xa, xb_), min2(ya, yb), min2(za, zb));
-            const float hi = min3(max2(xa, xb_), max2(ya, yb), max2(za, zb));
-            a += lo < hi ? (hi - lo) * rlen[r] : 0.0f;
-          }
-        }
-        a /= float(nr);
-        if (a != 0.0f) {
-          float ctr[3];
-          voxel_centre(A.G.g, ix, iy, iz, ctr);
-          if (!(distance_point_line(p0, p1, ctr) < A.G.sumRadii)) a = 0.0f;
-        }
+    return n;
+  };
+  // value of a voxel: mean over the rays of its bits, 0 outside the cull
+  auto sample = [&](int v, unsigned m) -> float {
+    float a = 0.0f;
+    const int ix = int(fdiv(uint32_t(v), A.div_yz));
+    const int rem = v - ix * int(A.div_yz.d);
+    const int iy = int(fdiv(uint32_t(rem), A.div_z));
+    const int iz = rem - iy * nz;
+    // (byte offsets below 2^24: a full-rate multiplication)
+    const char* ax = reinterpret_cast<const char*>(alpha + ix);
+    const char* ay = reinterpret_cast<const char*>(alpha + off1 + iy);
+    const char* az = reinterpret_cast<const char*>(alpha + off2 + iz);
+    const char* al = reinterpret_cast<const char*>(alpha + pl);
+    while (m) {
+      const int b = __ffs(int(m)) - 1;
+      m &= m - 1u;
+      const int r0 = ONE ? b : b * A.rpb;
+      const int r1 = ONE ? b + 1 : (r0 + A.rpb < nr ? r0 + A.rpb : nr);
+      for (int r = r0; r < r1; ++r) {
+        const unsigned o = __umul24(unsigned(r), 4u * unsigned(stride));
+        const float* x = reinterpret_cast<const float*>(ax + o);
+        const float* y = reinterpret_cast<const float*>(ay + o);
+        const float* z = reinterpret_cast<const float*>(az + o);
+        const float xa = x[0], xe = x[1], ya = y[0], ye = y[1], za = z[0], ze = z[1];
+        const float lo = max3(min2(xa, xe), min2(ya, ye), min2(za, ze));
+        const float hi = min3(max2(xa, xe), max2(ya, ye), max2(za, ze));
+        a += max2(hi - lo, 0.0f) * *reinterpret_cast<const float*>(al + o);
       }
-      const bool nzv = a != 0.0f;
-      if (MODE == kModeColsum) {
-        if (nzv) {
-          if (A.colsum_fx)
+    }
+    a /= float(nr);
+    if (cull && a != 0.0f) {
+      float end[3] = {p1[0], p1[1], p1[2]}, ctr[3];
+      // (keeps the line's length in here: few channels need it)
+      asm volatile("" : "+v"(end[0]), "+v"(end[1]), "+v"(end[2]));
+      voxel_centre(A.G.g, ix, iy, iz, ctr);
+      if (!(distance_point_line(p0, end, ctr) < A.G.sumRadii)) a = 0.0f;
+    }
+    return a;
+  };
+  for (int xb = 0; xb < nx; xb += kWave) {
+    // every wave makes the same prefix (and writes the same words)
+    int area = 0, wz = 0;
+    const int x = xb + lane;
+    if (x < nx && yhi[x] >= ylo[x]) {
+      wz = zhi[x] - zlo[x] + 1;
+      area = (yhi[x] - ylo[x] + 1) * wz;
+    }
+    const int incl = wave_inclusive_scan(area);
+    const int tot = __shfl(incl, kWave - 1, kWave);
+    if (tot == 0) continue;
+    s_pre[lane] = incl - area;
+    s_wz[lane] = wz;
+    wave_lds_fence();
+    const int nseg = (tot + kMRow - 1) / kMRow;
+    const int seg = (tot + nseg - 1) / nseg;
+    const int part = (seg + NW - 1) / NW;
+    for (int s0 = 0; s0 < tot; s0 += seg) {
+      const int s1 = s0 + seg < tot ? s0 + seg : tot;
+      const int k0 = s0 + w * part < s1 ? s0 + w * part : s1;
+      const int k1 = k0 + part < s1 ? k0 + part : s1;
+      const int n = list_items(k0, k1, xb);
+      if (lane == 0) s_wn[w] = n;
+      __syncthreads();
+      int all = 0;
+      for (int ww = 0; ww < NW; ++ww) all += s_wn[ww];
+      // voxels in order of their number of bits: the lanes of a wave then
+      // loop alike (in list order a wave ran 3.9 times its mean)
+      const int bin = lane < 32 ? s_bin[lane] : 0;
+      const int first = wave_inclusive_scan(bin) - bin;
+      for (int c = lane; c - lane < n; c += kWave) {
+        const int bb = c < n ? 32 - __popc(wb[c]) : 0;
+        const int f = __shfl(first, bb, kWave);
+        if (c < n) s_ord[f + atomicAdd(&s_place[bb], 1)] = (unsigned short)(w * CH + c);
+      }
+      __syncthreads();
+      if (t < 32) s_bin[t] = s_place[t] = 0;
+      for (int c = t; c < all; c += NT) {
+        const int j = s_ord[c];
+        const float a = sample(l_vox[j], l_bit[j]);
+        if (MODE == kModeCount)
+          count += a != 0.0f ? 1 : 0;
+        else
+          l_bit[j] = __float_as_uint(a);
+      }
+      if (MODE == kModeFill && t == 0) {
+        const int64_t end = int64_t(room) + vox_all;
+        s_off = end <= A.st_cap ? int64_t(staging_area(A, rl)) * A.st_cap + int64_t(room) : -1;
+      }
+      __syncthreads();
+      if (MODE == kModeColsum || MODE == kModeFwd) {
+        // in list order: neighbouring lanes, neighbouring voxels
+        for (int c = lane; c < n; c += kWave) {
+          const float a = __uint_as_float(wb[c]);
+          const int v = wv[c];
+          if (a == 0.0f) continue;
+          if (MODE == kModeFwd)
+            proj += double(a) * double(A.xin[v]);
+          else if (A.colsum_fx)
             atomicAdd(&A.colsum_fx[v], (unsigned long long)llrint(double(a) * A.fx_scale));
           else if (wt != 0.0)
             atomicAdd(&A.colsum[v], double(a) * wt);
         }
-      } else if (MODE == kModeFwd) {
-        if (nzv) proj += double(a) * double(A.xin[v]);
-      } else {
-        const uint64_t b = __ballot(nzv);
-        if (MODE == kModeFill && nzv) {
-          // positions only move down, and every lane has read its own
-          const int pos = kept + __popcll(b & lanemask_lt());
-          wv[pos] = v;
-          wb[pos] = __float_as_uint(a);
-        }
-        kept += __popcll(b);
       }
-      wave_lds_fence();
-    }
-    return kept;
-  };
-  for (int xb = 0; xb < nx; xb += kSmBlock) {
-    const int xn = nx - xb < kSmBlock ? nx - xb : kSmBlock;
-    int area = 0, wz = 0;
-    if (t < xn && yhi[xb + t] >= ylo[xb + t]) {
-      wz = zhi[xb + t] - zlo[xb + t] + 1;
-      area = (yhi[xb + t] - ylo[xb + t] + 1) * wz;
-    }
-    int tot;
-    const int pre = block_exclusive_scan<int, kSmBlock>(area, s_scan, &tot);
-    if (t < xn) {
-      s_rect[t][0] = ylo[xb + t];
-      s_rect[t][1] = zlo[xb + t];
-      s_rect[t][2] = wz;
-      s_rect[t][3] = pre;
-    }
-    __syncthreads();
-    if (MODE != kModeFill) {
-      // waves take chunks in turn; their order does not matter
-      for (int k = w * kMChunk; k < tot; k += kMRow)
-        count += wave_items(k, k + kMChunk < tot ? k + kMChunk : tot, xb, xn);
-      __syncthreads();
-    } else {
-      const int nseg = (tot + kMRow - 1) / kMRow;
-      const int seg = nseg ? (tot + nseg - 1) / nseg : 0;
-      const int part = (seg + kMWaves - 1) / kMWaves;
-      for (int s0 = 0; s0 < tot; s0 += seg) {
-        const int s1 = s0 + seg < tot ? s0 + seg : tot;
-        const int k0 = s0 + w * part < s1 ? s0 + w * part : s1;
-        const int k1 = k0 + part < s1 ? k0 + part : s1;
-        const int n = wave_items(k0, k1, xb, xn);
-        if (lane == 0) s_wn[w] = n;
+      if (MODE == kModeFill) {
+        // non-zero entries in list order into the row's staging
+        int kept = 0;
+        for (int c = lane; c - lane < n; c += kWave)
+          kept += __popcll(__ballot(c < n && wb[c] << 1 != 0u));
+        if (lane == 0) s_kept[w] = kept;
         __syncthreads();
-        int wpre = 0, all = 0;
-        for (int ww = 0; ww < kMWaves; ++ww) {
-          wpre += ww < w ? s_wn[ww] : 0;
-          all += s_wn[ww];
+        int wpre = 0, sum = 0;
+        for (int ww = 0; ww < NW; ++ww) {
+          wpre += ww < w ? s_kept[ww] : 0;
+          sum += s_kept[ww];
         }
-        if (rb_n + all > kMRow) flush();
-        for (int c = lane; c < n; c += kWave) {
-          rb_col[rb_n + wpre + c] = wv[c];
-          rb_val[rb_n + wpre + c] = __uint_as_float(wb[c]);
+        const int64_t off = s_off;
+        for (int c = lane; c - lane < n; c += kWave) {
+          const unsigned a = c < n ? wb[c] : 0u;
+          const uint64_t b = __ballot(a << 1 != 0u);
+          if (off >= 0 && a << 1 != 0u) {
+            const int64_t pos = off + row_n + wpre + __popcll(b & lanemask_lt());
+            A.st_col[pos] = wv[c];
+            A.st_val[pos] = __uint_as_float(a);
+          }
+          wpre += __popcll(b);
         }
-        rb_n += all;
-        __syncthreads();
+        row_n += sum;
       }
+      // the lists and counts are written again
+      if (s1 < tot || xb + kWave < nx) __syncthreads();
     }
   }
-  if (MODE == kModeFill) {
-    if (rb_n > 0) flush();
-    if (t == 0) A.row_nnz[rl] = flushed;
-    if (t == 0 && flushed == 0) A.pieces[rl] = Piece{rl, 0, 0, 0, 0};
+  if (MODE == kModeFill && t == 0) {
+    if (vox_all && s_off < 0) atomicOr(A.flags, 1u);
+    A.row_nnz[rl] = row_n;
+    A.pieces[rl] = Piece{rl, 0, vox_all ? s_off : 0, row_n, 0};
   }
   if (MODE == kModeCount) {
-    if (lane == 0) s_wn[w] = count;
+    count = wave_reduce_sum(count);
+    if (lane == 0) s_kept[w] = count;
     __syncthreads();
     if (t == 0) {
       int n = 0;
-      for (int ww = 0; ww < kMWaves; ++ww) n += s_wn[ww];
+      for (int ww = 0; ww < NW; ++ww) n += s_kept[ww];
       A.row_nnz[rl] = n;
     }
   }
@@ -879,7 +1009,7 @@ __global__ __launch_bounds__(kSmBlock) void k_sm_rays(BuildArgs A) {
     __syncthreads();
     if (t == 0) {
       double tot = 0.0;
-      for (int ww = 0; ww < kMWaves; ++ww) tot += s_red[ww];
+      for (int ww = 0; ww < NW; ++ww) tot += s_red[ww];
       A.fwd[li] = tot;
     }
   }
@@ -942,8 +1072,27 @@ int make_build_args(const raptr_setup_t* setup, const raptr_grid_t* grid, int nr
   A->seed = seed;
   A->raygen = raygen;
   A->pl = grid->n[0] + grid->n[1] + grid->n[2] + 3;
-  A->div_x = make_fastdiv(uint32_t(grid->n[0]));
-  A->div_pl = make_fastdiv(uint32_t(A->pl));
+  uint32_t per = uint32_t(setup->n1y);
+  A->div_c[3] = make_fastdiv(per);
+  A->div_c[2] = make_fastdiv(per *= uint32_t(setup->n1z));
+  A->div_c[1] = make_fastdiv(per *= uint32_t(setup->n0y));
+  A->div_c[0] = make_fastdiv(per *= uint32_t(setup->n0z));
+  A->plain_planes = true;
+  for (int d = 0; d < 3; ++d) {
+    A->inv_d[d] = 1.0f / grid->d[d];
+    A->ext[d] = std::fabs(grid->o[d]) + float(grid->n[d]) * grid->d[d];
+    A->plain_planes = A->plain_planes && plain_size(grid->o[d], 60) && plain_size(grid->d[d], 59);
+  }
+  // the cull's radius less half a voxel's diagonal and the rounding error of
+  // its test (the cross product's terms are of the heads' distance squared)
+  const float heads = std::fabs(setup->pos1x - setup->pos0x) +
+                      float(setup->n0z + setup->n1z) * setup->segz +
+                      float(setup->n0y + setup->n1y) * setup->segy;
+  const float near = A->G.sumRadii * 0.9999f -
+                     0.5f * std::sqrt(grid->d[0] * grid->d[0] + grid->d[1] * grid->d[1] +
+                                      grid->d[2] * grid->d[2]) -
+                     2e-6f * (heads + A->ext[0] + A->ext[1] + A->ext[2]);
+  A->near2 = near > 0.0f ? near * near : 0.0f;
   A->rpb = (nrays + 31) / 32;
   *lds = build_lds_bytes(nrays, A->pl);
   if (*lds > 160 * 1024)
@@ -952,19 +1101,20 @@ int make_build_args(const raptr_setup_t* setup, const raptr_grid_t* grid, int nr
   return RAPTR_OK;
 }
 
-size_t rays_lds_bytes(const BuildArgs& A, bool fill) {
+size_t rays_lds_bytes(const BuildArgs& A) {
   const size_t nsm = A.G.g.n[0] > A.G.g.n[2] ? A.G.g.n[0] : A.G.g.n[2];
-  return 4 * (size_t(A.nrays) * (9 + size_t(A.pl)) + 2 * nsm * kMw + 4 * size_t(A.G.g.n[0]) +
-              size_t(kMRow) * (fill ? 4 : 2));
+  const size_t lists = 2 * size_t(kMRow), rays = 16 * size_t(A.nrays);
+  return 4 * (size_t(A.nrays) * ((size_t(A.pl) + 1) | 1) + 2 * nsm * kMw + 4 * size_t(A.G.g.n[0]) +
+              (lists > rays ? lists : rays));
 }
 
 template <class K>
-int launch_rows(K kernel, const BuildArgs& A, size_t lds, hipStream_t st) {
+int launch_rows(K kernel, const BuildArgs& A, size_t lds, hipStream_t st, int threads = kSmBlock) {
   // Raise the dynamic-LDS limit; not fatal where the default suffices.
   if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                           160 * 1024) != hipSuccess)
     (void)hipGetLastError();
-  hipLaunchKernelGGL(kernel, dim3(unsigned(A.rows)), dim3(kSmBlock), lds, st, A);
+  hipLaunchKernelGGL(kernel, dim3(unsigned(A.rows)), dim3(threads), lds, st, A);
   RAPTR_LAUNCH_CHECK();
   return RAPTR_OK;
 }
@@ -975,11 +1125,17 @@ int launch_rows(K kernel, const BuildArgs& A, size_t lds, hipStream_t st) {
 // buffers are smaller than they).
 template <int MODE>
 int launch_build(const BuildArgs& A, size_t lds, hipStream_t st) {
-  const size_t lr = rays_lds_bytes(A, MODE == kModeFill) + 8192;  // + static
-  if (A.raygen == RAPTR_RAYGEN_RAND_ELEMENT || A.keep_zeros || lr > 160 * 1024)
+  const size_t lr = rays_lds_bytes(A);
+  if (A.by_candidate || A.raygen == RAPTR_RAYGEN_RAND_ELEMENT || A.keep_zeros || lr > 156 * 1024 ||
+      int64_t(A.G.g.n[0]) * A.G.g.n[1] >= 1 << 24)
     return launch_rows(k_sm_build<MODE>, A, lds, st);
-  if (A.rpb == 1) return launch_rows(k_sm_rays<MODE, true>, A, lr - 8192, st);
-  return launch_rows(k_sm_rays<MODE, false>, A, lr - 8192, st);
+  // Two waves a row where the rays' tables are small, four else: a wave's
+  // share of each phase must outlast the barriers.  147,456 rows of 10 rays x
+  // 99 planes: 0.96 ms with two, 1.02 with four; 40,009 of 17 x 131: 1.04 and
+  // 0.98; 100,003 of 30 x 159: 2.23 and 1.78 (8 waves: 2.24).
+  if (A.rpb > 1) return launch_rows(k_sm_rays<MODE, false, 4>, A, lr, st, 256);
+  if (A.nrays * A.pl < 1536) return launch_rows(k_sm_rays<MODE, true, 2>, A, lr, st, 128);
+  return launch_rows(k_sm_rays<MODE, true, 4>, A, lr, st, 256);
 }
 
 // Workspace layout of the fused build for a staging area of S entries:
@@ -1120,7 +1276,9 @@ int raptr_sm_build_csr_ex(const raptr_setup_t* setup, const raptr_grid_t* grid,
 
   int64_t total = 0;
   int first = 0;
-  double share = 0.7;  // of the staging that a chunk should fill
+  // of the staging that a chunk's entries should fill (k_sm_rays asks for a
+  // fourth to a half more than they)
+  double share = 0.6;
   // the first chunk measures the density: rows of up to 4,096 entries fit
   int64_t rows0 = staging >> 12;
   if (rows0 < 64) rows0 = 64;
@@ -1152,12 +1310,18 @@ int raptr_sm_build_csr_ex(const raptr_setup_t* setup, const raptr_grid_t* grid,
     RAPTR_HIP_TRY(hipMemcpyAsync(hc, counters, sizeof(hc), hipMemcpyDeviceToHost, st));
     RAPTR_HIP_TRY(hipStreamSynchronize(st));
     if (unsigned(hc[1] & 0xffffffffu)) {
-      if (rows == 1)
-        return fail(RAPTR_ERR_WORKSPACE, "row %d does not fit the staging area", first);
+      if (rows == 1) {
+        // k_sm_rays asks for room for its rectangles, k_sm_build for entries
+        if (A.by_candidate)
+          return fail(RAPTR_ERR_WORKSPACE, "row %d does not fit the staging area", first);
+        A.by_candidate = 1;
+        continue;
+      }
       rows = rows / 2;
       share *= 0.5;
       continue;
     }
+    A.by_candidate = 0;
     const int64_t chunk_nnz = int64_t(hc[2]);
     if (fill) {
       if (total + chunk_nnz > capacity)

@@ -108,7 +108,7 @@ class DeviceCSR:
         return self.nnz * (self.val.dtype.itemsize + 4) + (self.m + 1) * 8
 
 
-DEFAULT_STAGING = 64 << 20  # staging entries of the chunked build
+DEFAULT_STAGING = 64 << 20  # staging entries of the chunked build, at most
 
 
 def build_csr(setup, grid, cnl_list, nrays, seed=1, raygen=capi.RAYGEN_RAND, stream=None,
@@ -126,6 +126,10 @@ def build_csr(setup, grid, cnl_list, nrays, seed=1, raygen=capi.RAYGEN_RAND, str
         d_list = DeviceArray.from_numpy(lst)
     s, g = setup.struct(), grid.struct()
     L = capi.lib()
+    if not keep_zeros and raygen != capi.RAYGEN_RAND_ELEMENT:
+        # 16M entries hold some 20,000 rows at a time, enough to fill the
+        # device; a larger area costs more to allocate than it saves
+        staging = min(int(staging), max(16 << 20, grid.nvox))
     ws = Workspace(L.raptr_sm_build_workspace_size(C.byref(g), int(nrays), int(staging)))
     rp = DeviceArray(m + 1, np.int64)
     nnz = C.c_int64()
