@@ -355,9 +355,10 @@ int raptr_mlem_partial_slots(int n);
  * (64-bit row pointers, ascending columns) and the FP64 sensitivity.  The
  * plan owns two derived layouts: a row-padded CSR (16-byte aligned rows,
  * vector loads) for the forward pass and the transpose cut into row blocks
- * of block_rows channels (0: 65,536 for single-frame row-blocked plans,
- * else sized so the block's 2 MB ratio slice fits one XCD's L2) for the
- * atomic-free backward pass.  value_type: 0 = FP32,
+ * of block_rows channels (0: 65,536 for single-frame row-blocked plans, a
+ * multiple of 8 blocks of at most 16,384 rows for 64 frames, else sized so
+ * the block's 2 MB ratio slice fits one XCD's L2) for the atomic-free
+ * backward pass.  value_type: 0 = FP32,
  * 1 = FP16, 2 = BF16 (of value/row maximum), 3 = UNORM16 (fixed point
  * round(65535*value/row maximum)); 16-bit types carry a per-row FP32
  * scale and accumulate in FP32.  max_frames: batch capacity (power of two <= 64).  The
@@ -540,7 +541,8 @@ int raptr_recon_get_fused(const raptr_recon* plan, int* available, int* on, int*
  *   0: all of a column's group partials in one pass, by column;
  *   1: the groups split into 8 ranges, one per XCD (workgroup i runs on
  *      XCD i % 8), so each XCD's L2 holds an eighth of the partial sums;
- *      the 8 range sums of a column added in order;
+ *      the 8 range sums of a column added in order (plans of fewer than 128
+ *      union entries per column: one pass by column, as mode 0);
  *   2 (the default where the plan's segment table gives at least 512
  *      workgroups; else 1): column tiles:
  *      per part of a tile's groups, their partials read in the order the
@@ -642,8 +644,9 @@ int64_t raptr_recon_transpose_nnz(const raptr_recon* plan);
  * [n][nframes], start images in, results out.  Per frame and iteration:
  * yt = A x, e = y/yt (0 where y or yt is 0), c = A^T e,
  * x = x*c/(s + (s==0)), x *= 1/sum(x) (FP64 sum).  With use_graph and a
- * non-null stream the iteration is captured once into a HIP graph (cached
- * per frame count and buffers, raptr_recon_graph_count) and replayed. */
+ * non-null stream the iteration (small plans: also four in a row) is
+ * captured once into a HIP graph (cached per frame count and buffers,
+ * raptr_recon_graph_count) and replayed. */
 int raptr_recon_mlem(raptr_recon* plan, int nframes, const float* d_y, float* d_x,
                      int niter, int use_graph, raptr_stream_t stream);
 /* raptr_recon_mlem over the first `active` frames (16 or 32) of a 64-frame

@@ -1168,6 +1168,56 @@ __global__ __launch_bounds__(256) void k_fwdm64(int64_t ng, int64_t m,
   }
 }
 
+// k_fwdm64 with one group per workgroup: each wave sums a quarter of the
+// group's union list, and the waves' sums are added in wave order (a row's
+// ratio by the wave of its register).  For plans of at most kSplitGroups
+// groups, where one wave per group leaves a SIMD a few waves, waiting for
+// their gathers: 1,268 groups of 696 entries 85 -> 48 us (with the counts'
+// permutation), 2,484 of 2,200 301 -> 217; 8,826 of 465 191 and 189, 23,719 of
+// 1,280 1,106 and 1,137.
+constexpr int64_t kSplitGroups = 8192;
+template <int VT, int FB>
+__global__ __launch_bounds__(256) void k_fwdm64s(int64_t ng, int64_t m,
+                                                 const int64_t* __restrict__ gp,
+                                                 const int* __restrict__ gcol,
+                                                 const typename Val<VT>::T* __restrict__ gval,
+                                                 const float* __restrict__ rscale,
+                                                 const float* __restrict__ x,
+                                                 const float* __restrict__ y,
+                                                 float* __restrict__ e) {
+  using M = MF<16>;
+  constexpr int U = 4, E = M::K * U, NW = 256 / kWave;
+  __shared__ float part[NW][M::NR * FB][kWave];
+  const int lane = threadIdx.x & (kWave - 1), w = wave_id();
+  const int kq = lane / M::W, rw = lane % M::W;
+  const int64_t g = xcd_block(blockIdx.x, gridDim.x);
+  const int64_t b = gp[g], steps = (gp[g + 1] - b) / E;  // (lists are multiples of 32)
+  typename M::acc_t acc[FB];
+  acc_zero<16, FB>(acc);
+  mfma_sum<VT, 16, U, false, FB>(gcol, gval, b + E * (steps * w / NW),
+                                 b + E * (steps * (w + 1) / NW), x + FB * rw, kq, rw, acc);
+#pragma unroll
+  for (int r = 0; r < M::NR; ++r)
+#pragma unroll
+    for (int fb = 0; fb < FB; ++fb) part[w][r * FB + fb][lane] = acc[fb][r];
+  __syncthreads();
+  static_assert(M::NR == NW, "a wave finishes one register's rows");
+  const int64_t row = int64_t(16) * g + M::member(lane, w);
+  if (row >= m) return;
+  const float sc = VT == kF32 ? 1.0f : rscale[row];
+#pragma unroll
+  for (int fb = 0; fb < FB; ++fb) {
+    float sum = part[0][w * FB + fb][lane];
+#pragma unroll
+    for (int k = 1; k < NW; ++k) sum += part[k][w * FB + fb][lane];
+    const int64_t o = row * 64 + FB * rw + fb;
+    const float yy = y[o];
+    const float yt = sc * sum;
+    const float t = (yt != 0.0f && yy != 0.0f) ? yy / yt : 0.0f;
+    e[o] = VT == kF32 ? t : sc * t;  // ratio folded with the row scale
+  }
+}
+
 template <int VT, int U>
 __global__ __launch_bounds__(256) void k_bwdm64(int ngc, const int64_t* __restrict__ gp,
                                                 int nbl, const int* __restrict__ grow,
@@ -1286,26 +1336,33 @@ __global__ __launch_bounds__(256) void k_bwdm64x(int ngc, int nblk, int n,
 }
 
 // c = sum of the 8 partial images (XCD order), x' = x*c/(s + (s==0)), and
-// FP64 partial sums per workgroup (4 voxels) and frame; frames fa .. 63 are
-// skipped (x' and their partial sums not written)
-__global__ __launch_bounds__(256) void k_bwd_xreduce(int n, int fa, const float* __restrict__ c8,
+// FP64 partial sums per workgroup (4 * per voxels) and frame; frames fa .. 63
+// are skipped (x' and their partial sums not written).  per: voxels in turn,
+// so that some 2,048 rows of partial sums are left for k_norms (one row per
+// 4 voxels made 18 MB of them at 52^3: 62 us here and 67 there,
+// now 45 and 13).
+__global__ __launch_bounds__(256) void k_bwd_xreduce(int n, int fa, int per,
+                                                     const float* __restrict__ c8,
                                                      const float* __restrict__ x,
                                                      const float* __restrict__ s,
                                                      float* __restrict__ xx,
                                                      double* __restrict__ partials) {
   const int f = threadIdx.x & 63, jj = threadIdx.x >> 6;
-  const int64_t j = int64_t(blockIdx.x) * 4 + jj;
   double part = 0.0;
-  if (j < n && f < fa) {
-    float cv = 0.0f;
+  if (f < fa)
+#pragma unroll 2
+    for (int it = 0; it < per; ++it) {
+      const int64_t j = (int64_t(blockIdx.x) * per + it) * 4 + jj;
+      if (j >= n) break;
+      float cv = 0.0f;
 #pragma unroll
-    for (int q = 0; q < 8; ++q) cv += c8[(int64_t(q) * n + j) * 64 + f];
-    float d = s[j];
-    d += float(d == 0.0f);
-    const float nv = x[j * 64 + f] * cv / d;
-    xx[j * 64 + f] = nv;
-    part = double(nv);
-  }
+      for (int q = 0; q < 8; ++q) cv += c8[(int64_t(q) * n + j) * 64 + f];
+      float d = s[j];
+      d += float(d == 0.0f);
+      const float nv = x[j * 64 + f] * cv / d;
+      xx[j * 64 + f] = nv;
+      part += double(nv);
+    }
   __shared__ double red[4][64];
   red[jj][f] = part;
   __syncthreads();
@@ -1658,9 +1715,12 @@ __global__ __launch_bounds__(64 * W) void k_fb1l(int64_t m, int rows,
 // lane's terms in order, then a fixed tree over the lanes), then
 // x'_j = x_j c_j / (s_j + (s_j == 0)) and an FP64 partial sum per
 // workgroup.  Workgroups of one XCD take consecutive columns, whose
-// partials lie side by side in each group's sorted union.
+// partials lie side by side in each group's sorted union; each takes `per`
+// runs of 256 / LPC of them, so that at most about 2,048 partial sums are left
+// for k_norm_scale.
 template <int LPC, int U>
-__global__ __launch_bounds__(256) void k_fb1_reduce(int n, const int64_t* __restrict__ vptr,
+__global__ __launch_bounds__(256) void k_fb1_reduce(int n, int per,
+                                                    const int64_t* __restrict__ vptr,
                                                     const int* __restrict__ vpos,
                                                     const float* __restrict__ cpart,
                                                     const float* __restrict__ x,
@@ -1669,32 +1729,34 @@ __global__ __launch_bounds__(256) void k_fb1_reduce(int n, const int64_t* __rest
                                                     double* __restrict__ partials) {
   const int lane = int(threadIdx.x) % LPC;
   const int64_t blk = xcd_block(blockIdx.x, gridDim.x);
-  const int64_t j = blk * (256 / LPC) + int(threadIdx.x) / LPC;
-  float acc = 0.0f;
-  if (j < n) {
-    const int64_t k1 = vptr[j + 1];
-    int64_t k = vptr[j] + lane;
-    for (; k + int64_t(LPC) * (U - 1) < k1; k += int64_t(LPC) * U) {
-      int p[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) p[u] = vpos[k + LPC * u];
-      float g[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) g[u] = cpart[p[u]];
-#pragma unroll
-      for (int u = 0; u < U; ++u) acc += g[u];
-    }
-    for (; k < k1; k += LPC) acc += cpart[vpos[k]];
-  }
-#pragma unroll
-  for (int off = LPC / 2; off >= 1; off >>= 1) acc += __shfl_xor(acc, off, LPC);
   double part = 0.0;
-  if (j < n && lane == 0) {
-    float d = s[j];
-    d += float(d == 0.0f);
-    const float nv = x[j] * acc / d;
-    xx[j] = nv;
-    part = double(nv);
+  for (int it = 0; it < per; ++it) {
+    const int64_t j = (blk * per + it) * (256 / LPC) + int(threadIdx.x) / LPC;
+    float acc = 0.0f;
+    if (j < n) {
+      const int64_t k1 = vptr[j + 1];
+      int64_t k = vptr[j] + lane;
+      for (; k + int64_t(LPC) * (U - 1) < k1; k += int64_t(LPC) * U) {
+        int p[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) p[u] = vpos[k + LPC * u];
+        float g[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) g[u] = cpart[p[u]];
+#pragma unroll
+        for (int u = 0; u < U; ++u) acc += g[u];
+      }
+      for (; k < k1; k += LPC) acc += cpart[vpos[k]];
+    }
+#pragma unroll
+    for (int off = LPC / 2; off >= 1; off >>= 1) acc += __shfl_xor(acc, off, LPC);
+    if (j < n && lane == 0) {
+      float d = s[j];
+      d += float(d == 0.0f);
+      const float nv = x[j] * acc / d;
+      xx[j] = nv;
+      part += double(nv);
+    }
   }
   __shared__ double red[256];
   red[threadIdx.x] = part;
@@ -2230,6 +2292,35 @@ __global__ __launch_bounds__(256) void k_norms(const double* partials, int nb, i
   }
 }
 
+// One frame: k_norms and k_scale_frames in one launch.  Every workgroup adds
+// the partial sums itself, in k_norms' order (the same bits), then scales its
+// share of x'.  Two launches of 3 us each and the gap between them less, of 39
+// us per iteration at 32^3; up to kNormScaleMax partial sums (32 KiB from L2
+// per workgroup), where they take longer than a launch.
+constexpr int kNormScaleMax = 4096;
+__global__ __launch_bounds__(256) void k_norm_scale(const double* __restrict__ partials, int nb,
+                                                    int64_t n, const float* __restrict__ xx,
+                                                    float* scale, double* norm,
+                                                    float* __restrict__ x) {
+  __shared__ double red[256];
+  double t = 0.0;
+  for (int b = threadIdx.x; b < nb; b += 256) t += partials[b];
+  red[threadIdx.x] = t;
+  __syncthreads();
+  for (int s = 128; s > 0; s >>= 1) {
+    if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
+    __syncthreads();
+  }
+  const double tot = red[0];
+  const float sc = tot != 0.0 ? float(1.0 / tot) : 0.0f;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    norm[0] = tot;
+    scale[0] = sc;
+  }
+  for (int64_t j = int64_t(blockIdx.x) * 256 + threadIdx.x; j < n; j += int64_t(gridDim.x) * 256)
+    x[j] = sc * xx[j];
+}
+
 // x = scale * x' for frames 0 .. fa - 1 of each FR-frame row (the others
 // keep their values)
 __global__ void k_scale_frames(int64_t n, int FR, int fa, const float* xx, const float* scale,
@@ -2416,6 +2507,19 @@ int launch_fwd_any(const raptr_recon* R, int F, const float* x, const float* y, 
     const unsigned gg = unsigned((R->ngf + 3) / 4);
     const int GU = R->grp_unroll, GG = R->grp_g;
     const int FBA = R->fa / GG;
+    if (GG == 16 && R->ngf <= kSplitGroups) {
+#define RAPTR_M64S(VV, FB_)                                                                  \
+      if (R->vt == VV && FBA == FB_)                                                         \
+        hipLaunchKernelGGL((k_fwdm64s<VV, FB_>), dim3(unsigned(R->ngf)), dim3(256), 0, st,    \
+                           R->ngf, m, R->gfp, R->gfcol,                                      \
+                           (const typename Val<VV>::T*)R->gfval, R->rscale, x, y, e);
+#define RAPTR_M64SV(VV) RAPTR_M64S(VV, 4) RAPTR_M64S(VV, 2) RAPTR_M64S(VV, 1)
+      RAPTR_M64SV(kF32) RAPTR_M64SV(kF16) RAPTR_M64SV(kBF16) RAPTR_M64SV(kU16)
+#undef RAPTR_M64SV
+#undef RAPTR_M64S
+      RAPTR_LAUNCH_CHECK();
+      return RAPTR_OK;
+    }
 #define RAPTR_M64(VV, G_, UU, FB_)                                                           \
     if (R->vt == VV && GG == G_ && GU == MF<G_>::K * UU && FBA == FB_) {                     \
       hipLaunchKernelGGL((k_fwdm64<VV, G_, UU, FB_>), dim3(gg), dim3(256), 0, st, R->ngf, m,  \
@@ -2600,8 +2704,10 @@ int launch_bwd_xcd(const raptr_recon* R, const float* x, hipStream_t st, int* nb
     if (!launched) return fail(RAPTR_ERR_INVALID_ARG, "per-XCD backward shape unsupported");
     RAPTR_LAUNCH_CHECK();
   }
-  const unsigned nr = unsigned((int64_t(R->n) + 3) / 4);
-  hipLaunchKernelGGL(k_bwd_xreduce, dim3(nr), dim3(256), 0, st, R->n, R->fa,
+  const int64_t quads = (int64_t(R->n) + 3) / 4;
+  const int per = int((quads + 2047) / 2048);
+  const unsigned nr = unsigned((quads + per - 1) / per);
+  hipLaunchKernelGGL(k_bwd_xreduce, dim3(nr), dim3(256), 0, st, R->n, R->fa, per,
                      (const float*)R->c8, x, (const float*)R->s, R->xx, R->partials);
   RAPTR_LAUNCH_CHECK();
   if (nb_out) *nb_out = int(nr);
@@ -2719,7 +2825,12 @@ int launch_fused1(const raptr_recon* R, const float* x, const float* y, hipStrea
     if (nb_out) *nb_out = int(nr);
     return RAPTR_OK;
   }
-  if (R->fb_xcd) {
+  // Mode 1 splits a column's partials into eight ranges, one per XCD's L2;
+  // with fewer than 16 of them per column and range most of a column's lanes
+  // idle, and one pass by column is faster: 12.6 entries per column 5.1
+  // against 13.5 us, 47.6 24.6 against 63, 94 350 against 525; 277: 199
+  // against 165.
+  if (R->fb_xcd && R->lnu >= int64_t(128) * n) {
     const unsigned gg = unsigned(8 * ((int64_t(n) + (256 / L) - 1) / (256 / L)));
 #define RAPTR_FR8(LL)                                                                          \
   if (L == LL)                                                                                 \
@@ -2737,10 +2848,12 @@ int launch_fused1(const raptr_recon* R, const float* x, const float* y, hipStrea
     if (nb_out) *nb_out = int(nr);
     return RAPTR_OK;
   }
-  const unsigned nr = unsigned((int64_t(n) + (256 / L) - 1) / (256 / L));
+  const int64_t runs = (int64_t(n) + (256 / L) - 1) / (256 / L);
+  const int per = int((runs + 2047) / 2048);
+  const unsigned nr = unsigned((runs + per - 1) / per);
 #define RAPTR_FR(LL)                                                                           \
   if (L == LL)                                                                                 \
-    hipLaunchKernelGGL((k_fb1_reduce<LL, 4>), dim3(nr), dim3(256), 0, st, n,                    \
+    hipLaunchKernelGGL((k_fb1_reduce<LL, 4>), dim3(nr), dim3(256), 0, st, n, per,               \
                        (const int64_t*)R->vptr, (const int*)R->vpos, (const float*)R->cpart,   \
                        x, (const float*)R->s, R->xx, R->partials);
   RAPTR_FR(16) else RAPTR_FR(32) else RAPTR_FR(64) else return fail(RAPTR_ERR_INVALID_ARG,
@@ -2765,6 +2878,13 @@ int iteration(raptr_recon* R, int F, const float* y, float* x, hipStream_t st) {
     RAPTR_TRY(launch_fwd_any(R, F, x, y, R->e, st));
     for (int b = 0; b < R->nblk; b += R->bwd_bpl)
       RAPTR_TRY(launch_bwd_any(R, F, b, std::min(R->bwd_bpl, R->nblk - b), x, st, &nb));
+  }
+  if (F == 1 && nb <= kNormScaleMax) {
+    hipLaunchKernelGGL(k_norm_scale, dim3(grid_for(R->n, 1024, 256)), dim3(256), 0, st,
+                       (const double*)R->partials, nb, int64_t(R->n), (const float*)R->xx,
+                       R->scale, R->norm, x);
+    RAPTR_LAUNCH_CHECK();
+    return RAPTR_OK;
   }
   // active frames: all F, or the plan's fa of a 64-frame grouped pass
   const int FA = F == 64 && R->grp64 ? R->fa : F;
@@ -3385,8 +3505,19 @@ int create_plan(raptr_recon** out, int m, int n, int64_t nnz, const int64_t* d_r
   // single-frame row-blocked plans: 65,536 rows (256 KB slices, 16-bit
   // transpose rows; the per-XCD backward keeps an eighth of the blocks in
   // each XCD's L2)
-  if (block_rows <= 0)
+  if (block_rows <= 0) {
     block_rows = max_frames == 1 ? 65536 : std::max(1, (2 << 20) / (4 * max_frames));
+    // 64 frames: each XCD walks an eighth of the blocks, so a multiple of 8
+    // of them, of at most 16,384 rows (the launches' windows of rows are cut
+    // from them).  Backward with 3 blocks of 8,192 rows, as the 2 MiB slice
+    // alone gives 20,282 rows, 164 us, with 8 of 2,544 108 (16: 111); 141,209
+    // rows 18 blocks 357, 8 309, 16 320; 379,499 rows 47 blocks 930, 24 889,
+    // 16 879, 64 919.
+    if (max_frames == 64) {
+      const int64_t per = 8 * std::max<int64_t>(1, (int64_t(m) + 131071) / 131072);
+      block_rows = std::max(16, int((int64_t(m) + per - 1) / per + 15) / 16 * 16);
+    }
+  }
   R->blk_rows = block_rows;
   R->nblk = std::max(1, int((int64_t(m) + block_rows - 1) / block_rows));
   int rc;
@@ -4256,6 +4387,37 @@ int raptr_recon_mlem_active(raptr_recon* R, int nframes, int active, const float
   return rc;
 }
 
+// Iterations per replayed graph of small plans.  A replay costs the host
+// about 10 us and the device the gap to the next, as long as the kernels of
+// an iteration where a pass reads up to some 64M entries: five iterations of
+// 2.8M entries and one frame take 154 us with one per replay and 142 with four
+// (96 and 69 a call where three streams keep the device busy).
+constexpr int kGraphRun = 4;
+constexpr int64_t kGraphRunEntries = int64_t(64) << 20;
+
+static int capture_iterations(raptr_recon* R, int nframes, const float* d_y, float* d_x, int count,
+                              hipStream_t st, raptr_recon::CachedGraph& g, int k) {
+  hipGraph_t graph = nullptr;
+  RAPTR_HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+  int irc = RAPTR_OK;
+  for (int i = 0; i < count && !irc; ++i) irc = iteration(R, nframes, d_y, d_x, st);
+  const hipError_t ce = hipStreamEndCapture(st, &graph);
+  if (irc) {
+    if (graph) (void)hipGraphDestroy(graph);
+    return irc;
+  }
+  RAPTR_HIP_TRY(ce);
+  hipGraphExec_t exec = nullptr;
+  const hipError_t ie = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+  if (ie != hipSuccess) {
+    (void)hipGraphDestroy(graph);
+    return fail(RAPTR_ERR_DEVICE, "graph instantiate: %s", hipGetErrorString(ie));
+  }
+  g.graph[k] = graph;
+  g.exec[k] = exec;
+  return RAPTR_OK;
+}
+
 static int mlem_impl(raptr_recon* R, int nframes, const float* d_y, float* d_x, int niter,
                      int use_graph, hipStream_t st) {
   if (!valid_frames(nframes) || nframes > R->fmax)
@@ -4278,7 +4440,6 @@ static int mlem_impl(raptr_recon* R, int nframes, const float* d_y, float* d_x, 
   }
   const auto key = std::make_tuple(nframes, R->fa, uintptr_t(d_y), uintptr_t(d_x));
   auto it = R->graphs.find(key);
-  hipGraphExec_t exec = nullptr;
   if (it == R->graphs.end()) {
     if (R->graphs.size() >= kMaxGraphs) {
       auto lru = R->graphs.begin();
@@ -4289,26 +4450,22 @@ static int mlem_impl(raptr_recon* R, int nframes, const float* d_y, float* d_x, 
       destroy_graph(lru->second);
       R->graphs.erase(lru);
     }
-    hipGraph_t graph = nullptr;
-    RAPTR_HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-    int irc = iteration(R, nframes, d_y, d_x, st);
-    hipError_t ce = hipStreamEndCapture(st, &graph);
-    if (irc) {
-      if (graph) (void)hipGraphDestroy(graph);
-      return irc;
-    }
-    RAPTR_HIP_TRY(ce);
-    hipError_t ie = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-    if (ie != hipSuccess) {
-      (void)hipGraphDestroy(graph);
-      return fail(RAPTR_ERR_DEVICE, "graph instantiate: %s", hipGetErrorString(ie));
-    }
-    R->graphs[key] = {graph, exec, ++R->graph_tick};
-  } else {
-    exec = it->second.exec;
-    it->second.used = ++R->graph_tick;
+    it = R->graphs.emplace(key, raptr_recon::CachedGraph()).first;
   }
-  for (int i = 0; i < niter; ++i) RAPTR_HIP_TRY(hipGraphLaunch(exec, st));
+  it->second.used = ++R->graph_tick;
+  const int run = R->nnz * nframes <= kGraphRunEntries ? kGraphRun : 1;
+  for (int i = 0; i < niter;) {
+    const int k = run > 1 && niter - i >= run ? 1 : 0;
+    if (!it->second.exec[k]) {
+      const int rc = capture_iterations(R, nframes, d_y, d_x, k ? run : 1, st, it->second, k);
+      if (rc) {
+        if (!it->second.exec[0] && !it->second.exec[1]) R->graphs.erase(it);
+        return rc;
+      }
+    }
+    RAPTR_HIP_TRY(hipGraphLaunch(it->second.exec[k], st));
+    i += k ? run : 1;
+  }
   return RAPTR_OK;
 }
 

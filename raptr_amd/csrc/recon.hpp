@@ -201,10 +201,12 @@ struct raptr_recon {
   std::vector<size_t> asizes;  // bytes of allocs[i]
   // captured iterations, keyed by (frames, y, x) exactly; at most
   // kMaxGraphs, the least recently used destroyed first
+  // (exec[0]: one iteration, exec[1]: kGraphRun of them, each captured when it
+  // is first needed)
   struct CachedGraph {
-    hipGraph_t graph;
-    hipGraphExec_t exec;
-    uint64_t used;
+    hipGraph_t graph[2] = {nullptr, nullptr};
+    hipGraphExec_t exec[2] = {nullptr, nullptr};
+    uint64_t used = 0;
   };
   // keyed by (frames, active frames, y, x)
   std::map<std::tuple<int, int, uintptr_t, uintptr_t>, CachedGraph> graphs;
@@ -216,10 +218,12 @@ namespace raptr {
 constexpr size_t kMaxGraphs = 16;
 
 inline void destroy_graph(raptr_recon::CachedGraph& g) {
-  if (g.exec) (void)hipGraphExecDestroy(g.exec);
-  if (g.graph) (void)hipGraphDestroy(g.graph);
-  g.exec = nullptr;
-  g.graph = nullptr;
+  for (int k = 0; k < 2; ++k) {
+    if (g.exec[k]) (void)hipGraphExecDestroy(g.exec[k]);
+    if (g.graph[k]) (void)hipGraphDestroy(g.graph[k]);
+    g.exec[k] = nullptr;
+    g.graph[k] = nullptr;
+  }
 }
 
 // every captured iteration of the plan (after a change of kernel shape);
