@@ -269,6 +269,55 @@ __host__ __device__ inline float slab_length(const float* v, const float* r) {
   return (amax - amin) * sqrtf(dx * dx + dy * dy + dz * dz);
 }
 
+// The cull by voxel columns.  The centres of column (ix, iy) closer to a
+// channel's line than the radius form one z interval (a convex set meets a
+// line in an interval); it is found in FP64, widened by a relative radius slack
+// and one voxel at each end, so every voxel that passes the float test of the
+// reference lies in it.
+struct LineInterval {
+  float p0[3], p1[3];
+  double u0, u1, u2, qa, rr;
+  __device__ LineInterval(const Geom& G, int cnl) {
+    channel_centres(G, cnl, p0, p1);
+    u0 = double(p1[0]) - double(p0[0]);
+    u1 = double(p1[1]) - double(p0[1]);
+    u2 = double(p1[2]) - double(p0[2]);
+    const double len2 = u0 * u0 + u1 * u1 + u2 * u2;
+    const double il = len2 > 0.0 ? 1.0 / sqrt(len2) : 0.0;
+    u0 *= il;
+    u1 *= il;
+    u2 *= il;
+    rr = double(G.sumRadii) * (1.0 + 1e-4) + 1e-4;
+    qa = u0 * u0 + u1 * u1;
+  }
+  // number of voxels of the column that may pass, the first at lo
+  __device__ int column(const raptr_grid_t& g, int ix, int iy, int& lo) const {
+    const int nz = g.n[2];
+    const double ax = double(g.o[0]) + (ix + 0.5) * double(g.d[0]) - double(p0[0]);
+    const double ay = double(g.o[1]) + (iy + 0.5) * double(g.d[1]) - double(p0[1]);
+    const double sp = ax * u0 + ay * u1;
+    const double qc = ax * ax + ay * ay - sp * sp - rr * rr;
+    int hi = -1;
+    lo = 0;
+    if (qa < 1e-12) {
+      if (qc < 0.0) hi = nz - 1;
+    } else {
+      const double qb = -2.0 * sp * u2;
+      const double disc = qb * qb - 4.0 * qa * qc;
+      if (disc >= 0.0) {
+        const double sq = sqrt(disc);
+        const double z1 = double(p0[2]) + (-qb - sq) / (2.0 * qa);
+        const double z2 = double(p0[2]) + (-qb + sq) / (2.0 * qa);
+        const double f1 = (z1 - double(g.o[2])) / double(g.d[2]) - 0.5;
+        const double f2 = (z2 - double(g.o[2])) / double(g.d[2]) - 0.5;
+        lo = int(fmax(floor(f1) - 1.0, 0.0));
+        hi = int(fmin(ceil(f2) + 1.0, double(nz - 1)));
+      }
+    }
+    return hi >= lo ? hi - lo + 1 : 0;
+  }
+};
+
 // ------------------------------------------------------ device utils
 constexpr int kWave = 64;
 
