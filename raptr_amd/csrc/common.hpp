@@ -44,6 +44,12 @@ int fail(int code, const char* fmt, ...);
 
 inline hipStream_t S(raptr_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
 
+// ------------------------------------------------- device memory
+// hipMalloc and hipFree through a bounded cache of freed blocks (runtime.hip).
+// pool_free waits for the device, as hipFree does, unless the caller has.
+hipError_t pool_malloc(void** p, size_t bytes);
+hipError_t pool_free(void* p, bool idle = false);
+
 // ------------------------------------------------- workspace carving
 struct Carver {
   char* base;

@@ -2367,7 +2367,7 @@ int build_groups(raptr_recon* R, const L& lists, int64_t ng, int align, int64_t*
   z.take<int64_t>(4);
   z.take<char>(sb);
   void* tmp = nullptr;
-  hipError_t ae = hipMalloc(&tmp, z.bytes());
+  hipError_t ae = pool_malloc(&tmp, z.bytes());
   if (ae != hipSuccess) {
     (void)hipGetLastError();
     return fail(RAPTR_ERR_OUT_OF_MEMORY, "grouped layout scratch: %s", hipGetErrorString(ae));
@@ -2390,7 +2390,7 @@ int build_groups(raptr_recon* R, const L& lists, int64_t ng, int align, int64_t*
     (void)hipMemsetAsync(*gptr, 0, 8, st);
   }
   hipError_t se = hipStreamSynchronize(st);
-  (void)hipFree(tmp);
+  (void)pool_free(tmp);
   if (rc) return rc;
   if (se != hipSuccess) return fail(RAPTR_ERR_DEVICE, "grouped layout: %s", hipGetErrorString(se));
   *gnnz = h;
@@ -3140,7 +3140,7 @@ int build_local_columns(raptr_recon* R, hipStream_t st, int rows_req = 0) {
                        (const int64_t*)nullptr, (int*)nullptr, (uint16_t*)nullptr);
     void* tmp = nullptr;
     const size_t sb = scan_workspace_bytes(ng);
-    RAPTR_HIP_TRY(hipMalloc(&tmp, 512 + sb));
+    RAPTR_HIP_TRY(pool_malloc(&tmp, 512 + sb));
     int64_t* tot = static_cast<int64_t*>(tmp);
     rc = scan_exclusive_i64(cnt, R->lup, ng, tot, static_cast<char*>(tmp) + 256, sb, st);
     if (!rc) hipLaunchKernelGGL(k_set_last, dim3(1), dim3(1), 0, st, R->lup, int(ng),
@@ -3151,7 +3151,7 @@ int build_local_columns(raptr_recon* R, hipStream_t st, int rows_req = 0) {
     if (le == hipSuccess)
       le = hipMemcpyAsync(hc.data(), cnt, size_t(ng) * 8, hipMemcpyDeviceToHost, st);
     if (le == hipSuccess) le = hipStreamSynchronize(st);
-    (void)hipFree(tmp);
+    (void)pool_free(tmp);
     if (rc) return rc;
     if (le != hipSuccess)
       return fail(RAPTR_ERR_DEVICE, "column unions: %s", hipGetErrorString(le));
@@ -3198,7 +3198,7 @@ int build_tile_segments(raptr_recon* R, int tshift, int target, hipStream_t st) 
   z.take<uint32_t>(1);
   z.take<char>(scan_workspace_bytes(nu));
   void* tmp = nullptr;
-  hipError_t ae = hipMalloc(&tmp, z.bytes() + 4096);
+  hipError_t ae = pool_malloc(&tmp, z.bytes() + 4096);
   if (ae != hipSuccess) {
     (void)hipGetLastError();
     return fail(RAPTR_ERR_OUT_OF_MEMORY, "tile segments scratch: %s", hipGetErrorString(ae));
@@ -3238,7 +3238,7 @@ int build_tile_segments(raptr_recon* R, int tshift, int target, hipStream_t st) 
     z2.take<uint32_t>(size_t(nt) * 256);
     z2.take<uint32_t>(size_t(nt) * 256);
     z2.take<char>(scan_workspace_bytes(nt * 256));
-    ae = hipMalloc(&tmp2, z2.bytes() + 4096);
+    ae = pool_malloc(&tmp2, z2.bytes() + 4096);
     if (ae != hipSuccess) {
       (void)hipGetLastError();
       tmp2 = nullptr;
@@ -3276,8 +3276,8 @@ int build_tile_segments(raptr_recon* R, int tshift, int target, hipStream_t st) 
     }
   }
   (void)hipStreamSynchronize(st);
-  (void)hipFree(tmp);
-  if (tmp2) (void)hipFree(tmp2);
+  (void)pool_free(tmp);
+  if (tmp2) (void)pool_free(tmp2);
   // the workgroups: tile t's segments in ceil(count / target) parts of
   // equal size (one part for a tile with none)
   std::vector<int4> wg;
@@ -3372,7 +3372,7 @@ int build_union_index(raptr_recon* R, hipStream_t st) {
   z.take<uint32_t>(size_t(ntiles) * 256);
   z.take<char>(scan_workspace_bytes(ntiles * 256));
   void* tmp = nullptr;
-  hipError_t ae = hipMalloc(&tmp, z.bytes() + 4096);
+  hipError_t ae = pool_malloc(&tmp, z.bytes() + 4096);
   if (ae != hipSuccess) {
     (void)hipGetLastError();
     return fail(RAPTR_ERR_OUT_OF_MEMORY, "union index scratch: %s", hipGetErrorString(ae));
@@ -3400,7 +3400,7 @@ int build_union_index(raptr_recon* R, hipStream_t st) {
     if (le != hipSuccess) rc = fail(RAPTR_ERR_DEVICE, "union index: %s", hipGetErrorString(le));
   }
   (void)hipStreamSynchronize(st);
-  (void)hipFree(tmp);
+  (void)pool_free(tmp);
   if (rc) return rc;
   // the default single-frame iteration: one shared column-sum region, 64
   // lanes per row, the per-XCD reduce with 16 lanes per column; register-held
@@ -3536,7 +3536,7 @@ int create_plan(raptr_recon** out, int m, int n, int64_t nnz, const int64_t* d_r
     if (!go) {
       void* tmp = nullptr;
       size_t sb = scan_workspace_bytes(m);
-      RAPTR_HIP_TRY(hipMalloc(&tmp, size_t(m) * 8 + 512 + sb));
+      RAPTR_HIP_TRY(pool_malloc(&tmp, size_t(m) * 8 + 512 + sb));
       plen = static_cast<int64_t*>(tmp);
       tot = reinterpret_cast<int64_t*>(static_cast<char*>(tmp) + ((size_t(m) * 8 + 255) & ~size_t(255)));
       char* sws = reinterpret_cast<char*>(tot) + 256;
@@ -3552,7 +3552,7 @@ int create_plan(raptr_recon** out, int m, int n, int64_t nnz, const int64_t* d_r
       int64_t h = 0;
       (void)hipMemcpyAsync(&h, tot, 8, hipMemcpyDeviceToHost, st);
       (void)hipStreamSynchronize(st);
-      (void)hipFree(tmp);
+      (void)pool_free(tmp);
       if (rc) return bail(rc);
       R->pnnz = h;
     }
@@ -3611,7 +3611,7 @@ int create_plan(raptr_recon** out, int m, int n, int64_t nnz, const int64_t* d_r
       const size_t sb = scan_workspace_bytes(T);
       const size_t tb = ((size_t(T) + 1) * 8 + 255) & ~size_t(255);
       void* tmp = nullptr;
-      RAPTR_HIP_TRY(hipMalloc(&tmp, sort_ws + 2 * tb + 256 + sb));
+      RAPTR_HIP_TRY(pool_malloc(&tmp, sort_ws + 2 * tb + 256 + sb));
       // carve: rowid | key32 (unused) | sort buffers, in the order the
       // transpose helper lays them out, then the unpadded pointers, padded
       // lengths, scan total and scan scratch
@@ -3720,7 +3720,7 @@ int create_plan(raptr_recon** out, int m, int n, int64_t nnz, const int64_t* d_r
         if (!rc) R->grp64 = 1;
       }
       (void)hipStreamSynchronize(st);
-      (void)hipFree(tmp);
+      (void)pool_free(tmp);
       if (rc) return bail(rc);
     } else {
       (void)hipMemsetAsync(R->bptr, 0, sizeof(int64_t) * (size_t(T) + 1), st);
@@ -3857,7 +3857,7 @@ int raptr_recon_create_opts(raptr_recon** out, int m, int n, int64_t nnz, const 
   z.take<int>(size_t(nnz) + 1);
   z.take<float>(size_t(nnz) + 1);
   void* tmp = nullptr;
-  hipError_t ae = hipMalloc(&tmp, z.bytes());
+  hipError_t ae = pool_malloc(&tmp, z.bytes());
   if (ae != hipSuccess) {
     (void)hipGetLastError();
     return fail(RAPTR_ERR_OUT_OF_MEMORY, "row order scratch (%zu B): %s", z.bytes(),
@@ -3904,7 +3904,7 @@ int raptr_recon_create_opts(raptr_recon** out, int m, int n, int64_t nnz, const 
     rc = create_plan(out, m, n, nnz, prp, pcol, pval, d_sens, value_type, max_frames,
                      block_rows, o.layout, gdims, o.group, o.grouped_only, stream);
   (void)hipStreamSynchronize(st);
-  (void)hipFree(tmp);
+  (void)pool_free(tmp);
   if (rc) return rc;
   raptr_recon* R = *out;
   if ((rc = ralloc(R, &R->rperm, size_t(m) + 1)) ||
@@ -3968,7 +3968,7 @@ int raptr_locality_order_ex(const raptr_setup_t* setup, const int* d_channels, i
   z.take<uint32_t>(size_t(ntiles) * 256);
   z.take<char>(scan_workspace_bytes(ntiles * 256));
   void* tmp = nullptr;
-  hipError_t ae = hipMalloc(&tmp, z.bytes() + 4096);
+  hipError_t ae = pool_malloc(&tmp, z.bytes() + 4096);
   if (ae != hipSuccess) {
     (void)hipGetLastError();
     return fail(RAPTR_ERR_OUT_OF_MEMORY, "locality order scratch: %s", hipGetErrorString(ae));
@@ -3989,7 +3989,7 @@ int raptr_locality_order_ex(const raptr_setup_t* setup, const int* d_channels, i
     if (le != hipSuccess) rc = fail(RAPTR_ERR_DEVICE, "locality order: %s", hipGetErrorString(le));
   }
   (void)hipStreamSynchronize(st);
-  (void)hipFree(tmp);
+  (void)pool_free(tmp);
   return rc;
 }
 
@@ -3999,7 +3999,8 @@ int raptr_recon_destroy(raptr_recon* R) {
     return fail(RAPTR_ERR_INVALID_ARG, "plan has %d live clone(s): destroy them first",
                 R->nclones);
   clear_graphs(R);
-  for (void* p : R->allocs) (void)hipFree(p);
+  if (!R->allocs.empty()) (void)hipDeviceSynchronize();
+  for (void* p : R->allocs) (void)pool_free(p, true);
   if (R->parent) --R->parent->nclones;
   delete R;
   return RAPTR_OK;

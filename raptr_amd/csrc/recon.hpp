@@ -239,7 +239,7 @@ inline void clear_graphs(raptr_recon* R) {
 template <class T>
 int ralloc(raptr_recon* R, T** p, size_t count) {
   void* q = nullptr;
-  hipError_t e = hipMalloc(&q, std::max<size_t>(count * sizeof(T), 256));
+  hipError_t e = pool_malloc(&q, std::max<size_t>(count * sizeof(T), 256));
   if (e == hipErrorOutOfMemory) {
     (void)hipGetLastError();
     return fail(RAPTR_ERR_OUT_OF_MEMORY, "recon: out of device memory (%zu B)",
@@ -259,7 +259,7 @@ template <class T>
 void rfree(raptr_recon* R, T*& p) {
   for (size_t i = 0; p && i < R->allocs.size(); ++i) {
     if (R->allocs[i] != static_cast<void*>(p)) continue;
-    (void)hipFree(R->allocs[i]);
+    (void)pool_free(R->allocs[i]);
     R->bytes -= R->asizes[i];
     R->allocs.erase(R->allocs.begin() + i);
     R->asizes.erase(R->asizes.begin() + i);
