@@ -94,6 +94,13 @@ int scan_exclusive_u32(const uint32_t* in, uint32_t* out, int64_t n,
 int radix_sort_pairs(uint64_t* k0, uint64_t* k1, uint32_t* v0, uint32_t* v1, int64_t n,
                      int bits, hipStream_t st, int* result, Carver& cv);
 
+// The same with 64-bit values (32- or 64-bit keys); scratch of
+// sort_scratch_bytes(n) from cv.
+size_t sort_scratch_bytes(int64_t n);
+template <class K>
+int radix_sort_payload(K* k0, K* k1, uint64_t* v0, uint64_t* v1, int64_t n, int bits,
+                       hipStream_t st, int* result, Carver& cv);
+
 // Native vector types (accepted by the non-temporal load builtin).
 typedef float vf4 __attribute__((ext_vector_type(4)));
 typedef int vi4 __attribute__((ext_vector_type(4)));

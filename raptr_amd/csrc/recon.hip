@@ -109,27 +109,20 @@ __global__ __launch_bounds__(256) void k_row_scales(const int64_t* rp, const flo
   }
 }
 
-// transpose keys: (row block << colbits) | col, payload = entry index
-__global__ void k_bt_keys(const int64_t* rp, const int* col, int m, int blk_rows, int colbits,
-                          uint64_t* keys, uint32_t* idx) {
+// transpose keys: (row block << colbits) | col, payload: the row and the value
+template <class K>
+__global__ void k_bt_keys(const int64_t* rp, const int* col, const float* val, int m, int blk_rows,
+                          int colbits, K* keys, uint64_t* pay) {
   int64_t wid = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
   int lane = threadIdx.x & (kWave - 1);
   int64_t nw = int64_t(gridDim.x) * blockDim.x / kWave;
   for (int64_t i = wid; i < m; i += nw) {
-    uint64_t hi = uint64_t(i / blk_rows) << colbits;
+    const K hi = K(K(i / blk_rows) << colbits);
     for (int64_t k = rp[i] + lane; k < rp[i + 1]; k += kWave) {
-      keys[k] = hi | uint64_t(uint32_t(col[k]));
-      idx[k] = uint32_t(k);
+      keys[k] = hi | K(uint32_t(col[k]));
+      pay[k] = uint64_t(i) << 32 | uint64_t(__float_as_uint(val[k]));
     }
   }
-}
-
-__global__ void k_expand_rows32(const int64_t* rp, int m, uint32_t* rowid) {
-  int64_t wid = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
-  int lane = threadIdx.x & (kWave - 1);
-  int64_t nw = int64_t(gridDim.x) * blockDim.x / kWave;
-  for (int64_t i = wid; i < m; i += nw)
-    for (int64_t k = rp[i] + lane; k < rp[i + 1]; k += kWave) rowid[k] = uint32_t(i);
 }
 
 // padded segment lengths of the blocked transpose: segment (b, j) of
@@ -143,21 +136,25 @@ __global__ void k_bt_padlen(const int64_t* uptr, int64_t total, int n, int64_t* 
   }
 }
 
-// sorted entry j -> its place in the padded segment of its (block, column)
-__global__ void k_bt_scatter(const uint64_t* keys, const uint32_t* idx, int64_t nnz, int n,
+// sorted entry j -> its place in the padded segment of its (block, column);
+// brow16 (or null): the row's offset in its block
+template <class K>
+__global__ void k_bt_scatter(const K* keys, const uint64_t* pay, int64_t nnz, int n, int blk_rows,
                              int colbits, const int64_t* uptr, const int64_t* pptr,
-                             const uint32_t* rowid, const float* val, const float* scale,
-                             int vt, int* brow, void* bval, int C) {
-  const uint64_t cmask = (uint64_t(1) << colbits) - 1;
+                             const float* scale, int vt, int* brow, uint16_t* brow16, void* bval,
+                             int C) {
+  const K cmask = (K(1) << colbits) - 1;
   for (int64_t j = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; j < nnz;
        j += int64_t(gridDim.x) * blockDim.x) {
-    const uint64_t key = keys[j];
-    const int64_t t = int64_t(key >> colbits) * (n + 1) + int64_t(key & cmask);
+    const K key = keys[j];
+    const int64_t b = int64_t(key >> colbits);
+    const int64_t t = b * (n + 1) + int64_t(key & cmask);
     const int64_t d = pptr[t] + ilv(j - uptr[t], pptr[t + 1] - pptr[t], C);
-    const uint32_t k = idx[j];
-    const uint32_t r = rowid[k];
+    const uint64_t q = pay[j];
+    const uint32_t r = uint32_t(q >> 32);
     brow[d] = int(r);
-    const float v = val[k];
+    if (brow16) brow16[d] = uint16_t(r - uint32_t(b) * uint32_t(blk_rows));
+    const float v = __uint_as_float(uint32_t(q));
     if (vt == kF32)
       static_cast<float*>(bval)[d] = v;
     else
@@ -168,7 +165,7 @@ __global__ void k_bt_scatter(const uint64_t* keys, const uint32_t* idx, int64_t 
 
 // padding entries: value 0, row = the block's first row (inside the block)
 __global__ void k_bt_pad(const int64_t* uptr, const int64_t* pptr, int64_t total, int n,
-                         int blk_rows, int* brow, void* bval, int vt, int C) {
+                         int blk_rows, int* brow, uint16_t* brow16, void* bval, int vt, int C) {
   for (int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; t < total;
        t += int64_t(gridDim.x) * blockDim.x) {
     const int64_t b = t / (n + 1), j = t - b * (n + 1);
@@ -178,6 +175,7 @@ __global__ void k_bt_pad(const int64_t* uptr, const int64_t* pptr, int64_t total
     for (int64_t o = len; o < plen; ++o) {
       const int64_t p = pptr[t] + ilv(o, plen, C);
       brow[p] = int(b * blk_rows);
+      if (brow16) brow16[p] = 0;
       if (vt == kF32)
         static_cast<float*>(bval)[p] = 0.0f;
       else
@@ -188,7 +186,8 @@ __global__ void k_bt_pad(const int64_t* uptr, const int64_t* pptr, int64_t total
 
 // segment pointers of the blocked transpose: ptr[b*(n+1) + j] = first entry
 // with key >= (b << colbits | j)
-__global__ void k_bt_ptr(const uint64_t* keys, int64_t nnz, int nblk, int n, int colbits,
+template <class K>
+__global__ void k_bt_ptr(const K* keys, int64_t nnz, int nblk, int n, int colbits,
                          int64_t* ptr) {
   int64_t total = int64_t(nblk) * (n + 1);
   for (int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; t < total;
@@ -835,9 +834,7 @@ struct RowLists {
 template <int G>
 struct ColLists {
   const int64_t* uptr;
-  const uint32_t* idx;
-  const uint32_t* rowid;
-  const float* val;
+  const uint64_t* pay;  // row, value
   const int* cols;
   int n, ngc;
   __device__ void bounds(int64_t t, int64_t (&b)[G], int64_t (&e)[G]) const {
@@ -850,8 +847,8 @@ struct ColLists {
       e[s] = j >= 0 ? uptr[o + 1] : 0;
     }
   }
-  __device__ int key(int64_t k) const { return int(rowid[idx[k]]); }
-  __device__ float value(int64_t k) const { return val[idx[k]]; }
+  __device__ int key(int64_t k) const { return int(pay[k] >> 32); }
+  __device__ float value(int64_t k) const { return __uint_as_float(uint32_t(pay[k])); }
   __device__ int64_t row(int64_t, int, int key) const { return key; }
 };
 
@@ -2122,16 +2119,6 @@ __global__ void k_seq_cols(int n, int64_t total, int* __restrict__ cols) {
 
 // rows of the transpose as 16-bit offsets in their row block (blocks of at
 // most 65,536 rows): 6 bytes per FP32 entry instead of 8
-__global__ void k_bt_rows16(int64_t nb, int64_t bnnz, const int64_t* pptr, int n, int blk_rows,
-                            const int* brow, uint16_t* brow16) {
-  // one thread per (block, column) segment
-  for (int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; t < nb * (n + 1);
-       t += int64_t(gridDim.x) * blockDim.x) {
-    const int64_t b = t / (n + 1);
-    const int64_t r0 = b * blk_rows;
-    for (int64_t p = pptr[t]; p < pptr[t + 1]; ++p) brow16[p] = uint16_t(brow[p] - r0);
-  }
-}
 
 // forward columns as 16-bit low parts (grids of <= 4 x 65,536 voxels): one
 // wave per row; split[i] packs the row's first positions with a column >=
@@ -2330,18 +2317,35 @@ __global__ void k_scale_frames(int64_t n, int FR, int fa, const float* xx, const
     if (t % FR < fa) x[t] = scale[t % FR] * xx[t];
 }
 
-__global__ void k_sens_norm32(const double* sens, int n, float* s) {
+// s = sens / sum(sens) in FP32, the sum in FP64 over at most kSensSums parts in
+// a fixed order (one workgroup for all of it took 0.31 ms at 52^3, 2.2 at 96^3)
+constexpr int kSensSums = 256;
+__global__ __launch_bounds__(256) void k_sens_sum(const double* __restrict__ sens, int n,
+                                                  double* __restrict__ parts) {
   __shared__ double red[256];
   double t = 0.0;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) t += sens[i];
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += int(gridDim.x) * 256) t += sens[i];
   red[threadIdx.x] = t;
   __syncthreads();
-  for (int k = blockDim.x / 2; k > 0; k >>= 1) {
+  for (int k = 128; k > 0; k >>= 1) {
     if (threadIdx.x < k) red[threadIdx.x] += red[threadIdx.x + k];
     __syncthreads();
   }
-  double tot = red[0];
-  for (int i = threadIdx.x; i < n; i += blockDim.x) s[i] = float(sens[i] / tot);
+  if (threadIdx.x == 0) parts[blockIdx.x] = red[0];
+}
+__global__ __launch_bounds__(256) void k_sens_norm32(const double* __restrict__ sens, int n,
+                                                     const double* __restrict__ parts, int np,
+                                                     float* __restrict__ s) {
+  __shared__ double red[256];
+  red[threadIdx.x] = int(threadIdx.x) < np ? parts[threadIdx.x] : 0.0;
+  __syncthreads();
+  for (int k = 128; k > 0; k >>= 1) {
+    if (threadIdx.x < k) red[threadIdx.x] += red[threadIdx.x + k];
+    __syncthreads();
+  }
+  const double tot = red[0];
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += int(gridDim.x) * 256)
+    s[i] = float(sens[i] / tot);
 }
 
 }  // namespace
@@ -3088,56 +3092,77 @@ double union_model_ms(int64_t pnnz, int64_t entries, size_t lds) {
   const double rate = per_cu >= 3 ? 5.2e9 : per_cu == 2 ? 4.5e9 : 3.0e9;  // bytes per ms
   return (6.0 * double(pnnz) + 12.0 * double(entries)) / rate + 8.0 * double(entries) / 3.3e9;
 }
-int build_local_columns(raptr_recon* R, hipStream_t st, int rows_req = 0) {
+// (counted: the groups' union sizes on the device, where they are known already)
+int build_local_columns(raptr_recon* R, hipStream_t st, int rows_req = 0,
+                        int64_t* counted = nullptr) {
   const int64_t m = R->m;
   const int n = R->n;
   const size_t shm = (2 * size_t((std::min(n, kUnionWin) + 31) >> 5) + 257) * sizeof(uint32_t);
   int rc;
-  int64_t* cnt = nullptr;
+  int64_t* cnt = counted;
   int64_t h = 0, mx = 0;
   // without a request: the group sizes' union counts first (pass 0 each),
   // then the choice
   if (!rows_req) {
     const int nc = int(sizeof(kLocRowsChoices) / sizeof(int));
-    std::vector<double> cost(nc, 1e30);
+    // (sizes of too few groups are not counted; the smallest is the choice
+    // where no other has enough)
+    std::vector<int64_t> at(nc + 1, 0);
     for (int ci = 0; ci < nc; ++ci) {
-      const int rr = kLocRowsChoices[ci];
-      const int64_t ng = (m + rr - 1) / rr;
-      if ((rc = ralloc(R, &cnt, size_t(ng)))) return rc;
-      hipLaunchKernelGGL(k_loc_union, dim3(unsigned(ng)), dim3(256), shm, st,
-                         (const int64_t*)R->frp, (const int*)R->fcol, m, rr, n, 0, cnt,
-                         (const int64_t*)nullptr, (int*)nullptr, (uint16_t*)nullptr);
-      std::vector<int64_t> hc(static_cast<size_t>(ng));
+      const int64_t ng = (m + kLocRowsChoices[ci] - 1) / kLocRowsChoices[ci];
+      at[ci + 1] = at[ci] + (ng >= kMinGroups ? ng : 0);
+    }
+    int pick = nc - 1;
+    int64_t* all = nullptr;
+    if (at[nc] > 0) {
+      RAPTR_HIP_TRY(pool_malloc(reinterpret_cast<void**>(&all), size_t(at[nc]) * 8));
+      for (int ci = 0; ci < nc; ++ci)
+        if (at[ci + 1] > at[ci])
+          hipLaunchKernelGGL(k_loc_union, dim3(unsigned(at[ci + 1] - at[ci])), dim3(256), shm, st,
+                             (const int64_t*)R->frp, (const int*)R->fcol, m, kLocRowsChoices[ci],
+                             n, 0, all + at[ci], (const int64_t*)nullptr, (int*)nullptr,
+                             (uint16_t*)nullptr);
+      std::vector<int64_t> hc(static_cast<size_t>(at[nc]));
       hipError_t le = hipGetLastError();
       if (le == hipSuccess)
-        le = hipMemcpyAsync(hc.data(), cnt, size_t(ng) * 8, hipMemcpyDeviceToHost, st);
+        le = hipMemcpyAsync(hc.data(), all, size_t(at[nc]) * 8, hipMemcpyDeviceToHost, st);
       if (le == hipSuccess) le = hipStreamSynchronize(st);
-      rfree(R, cnt);
-      if (le != hipSuccess)
+      if (le != hipSuccess) {
+        (void)pool_free(all);
         return fail(RAPTR_ERR_DEVICE, "column unions: %s", hipGetErrorString(le));
-      const int64_t mxc = hc.empty() ? 0 : *std::max_element(hc.begin(), hc.end());
-      int64_t tot = 0;
-      for (int64_t v : hc) tot += v;
-      if (mxc <= kLocMaxUnion)
-        cost[ci] = union_model_ms(
-            R->pnnz, tot, size_t(rr + 1) * sizeof(int64_t) + size_t(2 * mxc + 1) * sizeof(float));
-    }
-    int pick = kLocRowsChoices[nc - 1];
-    double best = 1e30;
-    for (int ci = 0; ci < nc; ++ci)  // largest first: ties keep the larger groups
-      if ((m + kLocRowsChoices[ci] - 1) / kLocRowsChoices[ci] >= kMinGroups && cost[ci] < best) {
-        best = cost[ci];
-        pick = kLocRowsChoices[ci];
       }
-    return build_local_columns(R, st, pick);
+      double best = 1e30;
+      for (int ci = 0; ci < nc; ++ci) {  // largest first: ties keep the larger groups
+        int64_t tot = 0, mxc = 0;
+        for (int64_t i = at[ci]; i < at[ci + 1]; ++i) {
+          tot += hc[size_t(i)];
+          mxc = std::max(mxc, hc[size_t(i)]);
+        }
+        if (at[ci + 1] == at[ci] || mxc > kLocMaxUnion) continue;
+        const double cost = union_model_ms(
+            R->pnnz, tot,
+            size_t(kLocRowsChoices[ci] + 1) * sizeof(int64_t) + size_t(2 * mxc + 1) * sizeof(float));
+        if (cost < best) {
+          best = cost;
+          pick = ci;
+        }
+      }
+    }
+    rc = build_local_columns(R, st, kLocRowsChoices[pick],
+                             at[pick + 1] > at[pick] ? all + at[pick] : nullptr);
+    (void)pool_free(all);
+    return rc;
   }
   const int rows = rows_req;
   {
     const int64_t ng = (m + rows - 1) / rows;
-    if ((rc = ralloc(R, &R->lup, size_t(ng) + 1)) || (rc = ralloc(R, &cnt, size_t(ng)))) return rc;
-    hipLaunchKernelGGL(k_loc_union, dim3(unsigned(ng)), dim3(256), shm, st,
-                       (const int64_t*)R->frp, (const int*)R->fcol, m, rows, n, 0, cnt,
-                       (const int64_t*)nullptr, (int*)nullptr, (uint16_t*)nullptr);
+    if ((rc = ralloc(R, &R->lup, size_t(ng) + 1))) return rc;
+    if (!counted) {
+      if ((rc = ralloc(R, &cnt, size_t(ng)))) return rc;
+      hipLaunchKernelGGL(k_loc_union, dim3(unsigned(ng)), dim3(256), shm, st,
+                         (const int64_t*)R->frp, (const int*)R->fcol, m, rows, n, 0, cnt,
+                         (const int64_t*)nullptr, (int*)nullptr, (uint16_t*)nullptr);
+    }
     void* tmp = nullptr;
     const size_t sb = scan_workspace_bytes(ng);
     RAPTR_HIP_TRY(pool_malloc(&tmp, 512 + sb));
@@ -3607,56 +3632,57 @@ int create_plan(raptr_recon** out, int m, int n, int64_t nnz, const int64_t* d_r
       while ((int64_t(1) << colbits) <= n) ++colbits;
       int blkbits = 0;
       while ((int64_t(1) << blkbits) < R->nblk) ++blkbits;
-      const size_t sort_ws = raptr_csr_transpose_workspace_size(nnz, m, n);  // radix buffers
+      // 32-bit keys where block and column fit them
+      const bool k32 = colbits + blkbits <= 32;
+      const size_t kb = ((size_t(nnz) * (k32 ? 4 : 8)) + 255) & ~size_t(255);
+      const size_t pb = ((size_t(nnz) * 8) + 255) & ~size_t(255);
+      const size_t sort_ws = 2 * kb + 2 * pb + sort_scratch_bytes(nnz);
       const size_t sb = scan_workspace_bytes(T);
       const size_t tb = ((size_t(T) + 1) * 8 + 255) & ~size_t(255);
       void* tmp = nullptr;
       RAPTR_HIP_TRY(pool_malloc(&tmp, sort_ws + 2 * tb + 256 + sb));
-      // carve: rowid | key32 (unused) | sort buffers, in the order the
-      // transpose helper lays them out, then the unpadded pointers, padded
-      // lengths, scan total and scan scratch
+      // carve: keys, payloads and the sort's scratch, then the unpadded
+      // pointers, padded lengths, scan total and scan scratch
       Carver cv(tmp, sort_ws);
-      uint32_t* rowid = cv.take<uint32_t>(size_t(nnz));
-      (void)cv.take<int>(size_t(nnz));
-      rc = RAPTR_OK;
-      uint64_t* k0 = cv.take<uint64_t>(size_t(nnz));
-      uint64_t* k1 = cv.take<uint64_t>(size_t(nnz));
-      uint32_t* v0 = cv.take<uint32_t>(size_t(nnz));
-      uint32_t* v1 = cv.take<uint32_t>(size_t(nnz));
+      char* k0 = cv.take<char>(kb);
+      char* k1 = cv.take<char>(kb);
+      uint64_t* v0 = cv.take<uint64_t>(size_t(nnz));
+      uint64_t* v1 = cv.take<uint64_t>(size_t(nnz));
       char* extra = static_cast<char*>(tmp) + sort_ws;
       int64_t* uptr = reinterpret_cast<int64_t*>(extra);
       int64_t* plen = reinterpret_cast<int64_t*>(extra + tb);
       int64_t* tot = reinterpret_cast<int64_t*>(extra + 2 * tb);
       char* sws = extra + 2 * tb + 256;
-      if (!cv.ok) rc = fail(RAPTR_ERR_WORKSPACE, "transpose scratch carve failed");
-      uint64_t* keys = nullptr;
-      uint32_t* idx = nullptr;
-      int64_t h = 0;
-      if (!rc) {
-        hipLaunchKernelGGL(k_bt_keys, dim3(grid_for(int64_t(m) * kWave, 256, 1 << 16)), dim3(256),
-                           0, st, d_rp, d_col, m, block_rows, colbits, k0, v0);
-        hipLaunchKernelGGL(k_expand_rows32, dim3(grid_for(int64_t(m) * kWave, 256, 1 << 16)),
-                           dim3(256), 0, st, d_rp, m, rowid);
+      rc = cv.ok ? RAPTR_OK : fail(RAPTR_ERR_WORKSPACE, "transpose scratch carve failed");
+      const uint64_t* pay = nullptr;
+      const char* keys = nullptr;
+      auto sort_keys = [&](auto zero) -> int {
+        using K = decltype(zero);
+        K* a = reinterpret_cast<K*>(k0);
+        K* b = reinterpret_cast<K*>(k1);
+        hipLaunchKernelGGL(k_bt_keys<K>, dim3(grid_for(int64_t(m) * kWave, 256, 1 << 16)),
+                           dim3(256), 0, st, d_rp, d_col, d_val, m, block_rows, colbits, a, v0);
         int res = 0;
-        rc = radix_sort_pairs(k0, k1, v0, v1, nnz, colbits + blkbits, st, &res, cv);
-        if (!rc) {
-          keys = res ? k1 : k0;
-          idx = res ? v1 : v0;
-          hipLaunchKernelGGL(k_bt_ptr, dim3(grid_for(T, 256, 1 << 16)), dim3(256), 0, st,
-                             (const uint64_t*)keys, nnz, R->nblk, n, colbits, uptr);
-          if (!go) {
-            hipLaunchKernelGGL(k_bt_padlen, dim3(grid_for(T, 256, 1 << 16)), dim3(256), 0, st,
-                               (const int64_t*)uptr, T, n, plen);
-            rc = scan_exclusive_i64(plen, R->bptr, T, tot, sws, sb, st);
-          }
-        }
-        if (!rc && !go) {
-          hipLaunchKernelGGL(k_set_last, dim3(1), dim3(1), 0, st, R->bptr, int(T),
-                             (const int64_t*)tot);
-          (void)hipMemcpyAsync(&h, tot, 8, hipMemcpyDeviceToHost, st);
-          hipError_t se = hipStreamSynchronize(st);
-          if (se != hipSuccess) rc = fail(RAPTR_ERR_DEVICE, "transpose: %s", hipGetErrorString(se));
-        }
+        RAPTR_TRY(radix_sort_payload<K>(a, b, v0, v1, nnz, colbits + blkbits, st, &res, cv));
+        keys = res ? k1 : k0;
+        pay = res ? v1 : v0;
+        hipLaunchKernelGGL(k_bt_ptr<K>, dim3(grid_for(T, 256, 1 << 16)), dim3(256), 0, st,
+                           reinterpret_cast<const K*>(keys), nnz, R->nblk, n, colbits, uptr);
+        return RAPTR_OK;
+      };
+      int64_t h = 0;
+      if (!rc) rc = k32 ? sort_keys(uint32_t(0)) : sort_keys(uint64_t(0));
+      if (!rc && !go) {
+        hipLaunchKernelGGL(k_bt_padlen, dim3(grid_for(T, 256, 1 << 16)), dim3(256), 0, st,
+                           (const int64_t*)uptr, T, n, plen);
+        rc = scan_exclusive_i64(plen, R->bptr, T, tot, sws, sb, st);
+      }
+      if (!rc && !go) {
+        hipLaunchKernelGGL(k_set_last, dim3(1), dim3(1), 0, st, R->bptr, int(T),
+                           (const int64_t*)tot);
+        (void)hipMemcpyAsync(&h, tot, 8, hipMemcpyDeviceToHost, st);
+        hipError_t se = hipStreamSynchronize(st);
+        if (se != hipSuccess) rc = fail(RAPTR_ERR_DEVICE, "transpose: %s", hipGetErrorString(se));
       }
       if (!rc && !go) {
         R->bnnz = h;
@@ -3669,16 +3695,24 @@ int create_plan(raptr_recon** out, int m, int n, int64_t nnz, const int64_t* d_r
             if (!(rc = ralloc(R, &p, size_t(h) + 8))) R->bval = p;
           }
         }
+        // 16-bit row offsets in the block, beside the rows
+        if (!rc && max_frames == 1 && layout == RAPTR_LAYOUT_BLOCKED && block_rows <= 65536 && h > 0)
+          rc = ralloc(R, &R->brow16, size_t(h) + 8);
       }
       if (!rc && !go) {
-        hipLaunchKernelGGL(k_bt_scatter, dim3(grid_for(nnz, 256, 1 << 16)), dim3(256), 0, st,
-                           (const uint64_t*)keys, (const uint32_t*)idx, nnz, n, colbits,
-                           (const int64_t*)uptr, (const int64_t*)R->bptr,
-                           (const uint32_t*)rowid, d_val, (const float*)R->rscale, value_type,
-                           R->brow, R->bval, max_frames == 1 ? kIlvBwd : 0);
+        auto scatter = [&](auto zero) {
+          using K = decltype(zero);
+          hipLaunchKernelGGL(k_bt_scatter<K>, dim3(grid_for(nnz, 256, 1 << 16)), dim3(256), 0, st,
+                             reinterpret_cast<const K*>(keys), pay, nnz, n, block_rows, colbits,
+                             (const int64_t*)uptr, (const int64_t*)R->bptr,
+                             (const float*)R->rscale, value_type, R->brow, R->brow16, R->bval,
+                             max_frames == 1 ? kIlvBwd : 0);
+        };
+        if (k32) scatter(uint32_t(0)); else scatter(uint64_t(0));
         hipLaunchKernelGGL(k_bt_pad, dim3(grid_for(T, 256, 1 << 16)), dim3(256), 0, st,
                            (const int64_t*)uptr, (const int64_t*)R->bptr, T, n, block_rows,
-                           R->brow, R->bval, value_type, max_frames == 1 ? kIlvBwd : 0);
+                           R->brow, R->brow16, R->bval, value_type,
+                           max_frames == 1 ? kIlvBwd : 0);
         hipError_t le = hipGetLastError();
         if (le != hipSuccess) rc = fail(RAPTR_ERR_DEVICE, "transpose: %s", hipGetErrorString(le));
       }
@@ -3705,8 +3739,7 @@ int create_plan(raptr_recon** out, int m, int n, int64_t nnz, const int64_t* d_r
           switch (G) {
 #define RAPTR_CG(G_)                                                                       \
   case G_: {                                                                               \
-    ColLists<G_> L{(const int64_t*)uptr, (const uint32_t*)idx, (const uint32_t*)rowid,     \
-                   d_val, (const int*)R->gcols, n, int(R->ngc)};                           \
+    ColLists<G_> L{(const int64_t*)uptr, pay, (const int*)R->gcols, n, int(R->ngc)};       \
     rc = build_groups<G_>(R, L, int64_t(R->nblk) * R->ngc, kAlignBwd, &R->gbp, &R->gbrow,  \
                           &R->gbval, &R->gbnnz, st);                                       \
     break;                                                                                 \
@@ -3739,7 +3772,12 @@ int create_plan(raptr_recon** out, int m, int n, int64_t nnz, const int64_t* d_r
   if ((rc = ralloc(R, &R->partials, (size_t(n) / 4 + 8) * F))) return bail(rc);
   if ((rc = ralloc(R, &R->scale, size_t(F)))) return bail(rc);
   if ((rc = ralloc(R, &R->norm, size_t(F)))) return bail(rc);
-  hipLaunchKernelGGL(k_sens_norm32, dim3(1), dim3(256), 0, st, d_sens, n, R->s);
+  const int np = int(grid_for(n, 1024, kSensSums));
+  double* parts = nullptr;
+  if ((rc = ralloc(R, &parts, kSensSums))) return bail(rc);
+  hipLaunchKernelGGL(k_sens_sum, dim3(np), dim3(256), 0, st, d_sens, n, parts);
+  hipLaunchKernelGGL(k_sens_norm32, dim3(np), dim3(256), 0, st, d_sens, n, (const double*)parts,
+                     np, R->s);
   hipError_t le = hipGetLastError();
   if (le != hipSuccess) return bail(fail(RAPTR_ERR_DEVICE, "sens: %s", hipGetErrorString(le)));
   hipError_t se = hipStreamSynchronize(st);
@@ -3752,17 +3790,7 @@ int create_plan(raptr_recon** out, int m, int n, int64_t nnz, const int64_t* d_r
       (rc = ralloc(R, &R->c8, size_t(8) * n)))
     return bail(rc);
   // ... and the transpose's rows as 16-bit offsets in blocks of <= 65,536 rows
-  if (max_frames == 1 && layout == RAPTR_LAYOUT_BLOCKED && R->bptr && R->brow &&
-      block_rows <= 65536 && R->bnnz > 0) {
-    if ((rc = ralloc(R, &R->brow16, size_t(R->bnnz) + 8))) return bail(rc);
-    hipLaunchKernelGGL(k_bt_rows16, dim3(grid_for(int64_t(R->nblk) * (n + 1), 256, 1 << 16)),
-                       dim3(256), 0, st, int64_t(R->nblk), R->bnnz, (const int64_t*)R->bptr, n,
-                       block_rows, (const int*)R->brow, R->brow16);
-    hipError_t le = hipGetLastError();
-    if (le == hipSuccess) le = hipStreamSynchronize(st);
-    if (le != hipSuccess) return bail(fail(RAPTR_ERR_DEVICE, "rows16: %s", hipGetErrorString(le)));
-    R->bwd_r16 = 1;
-  }
+  if (R->brow16) R->bwd_r16 = 1;
   // ... and the forward's columns as 16-bit low parts (grids of <= 4 x 65,536
   // voxels, rows of <= 65,535 entries)
   if (max_frames == 1 && layout == RAPTR_LAYOUT_BLOCKED && R->fcol && int64_t(n) <= 4 * 65536 &&

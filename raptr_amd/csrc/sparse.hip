@@ -1,78 +1,117 @@
 // sparse.hip -- sparse-format kernels on gfx950: own stable LSD radix sort
 // (8-bit digits; per-tile histograms, device-wide scan, stable scatter with
-// wave-ballot peer ranking), COO sort, COO->CSR, CSR->ECSR, CSR transpose.
+// wave-ballot peer ranking through LDS), COO sort, COO->CSR, CSR->ECSR, CSR transpose.
 #include "primitives.hpp"
 
 namespace raptr {
 namespace {
 
 constexpr int kRsBlock = 256;
-constexpr int kRsRounds = 8;
-constexpr int kRsTile = kRsBlock * kRsRounds;
+constexpr int kRsItems = 16;  // per thread
+constexpr int kRsTile = kRsBlock * kRsItems;
 constexpr int kRsBins = 256;
 constexpr int kRsWaves = kRsBlock / kWave;
 
-__global__ __launch_bounds__(kRsBlock) void k_rs_hist(const uint64_t* keys, int64_t n,
-                                                      int shift, uint32_t* hist,
-                                                      int ntiles) {
+template <class K>
+__global__ __launch_bounds__(kRsBlock) void k_rs_hist(const K* keys, int64_t n, int shift,
+                                                      uint32_t* hist, int ntiles) {
   __shared__ uint32_t h[kRsBins];
   h[threadIdx.x] = 0;
   __syncthreads();
   int64_t base = int64_t(blockIdx.x) * kRsTile;
 #pragma unroll
-  for (int r = 0; r < kRsRounds; ++r) {
+  for (int r = 0; r < kRsItems; ++r) {
     int64_t p = base + r * kRsBlock + threadIdx.x;
-    if (p < n) atomicAdd(&h[(keys[p] >> shift) & 0xff], 1u);
+    if (p < n) atomicAdd(&h[uint32_t(keys[p] >> shift) & 0xff], 1u);
   }
   __syncthreads();
   hist[int64_t(threadIdx.x) * ntiles + blockIdx.x] = h[threadIdx.x];
 }
 
-// Stable scatter of one tile: rank = running count of the digit in earlier
-// rounds + counts of the digit in earlier waves of this round + rank among
-// equal-digit lanes of this wave (found with 8 ballots).
-__global__ __launch_bounds__(kRsBlock) void k_rs_scatter(const uint64_t* kin,
-                                                         const uint32_t* vin, int64_t n,
+// Stable scatter of one tile.  A wave takes 1,024 consecutive pairs, 64 at a
+// time: a pair's rank is the wave's running count of its digit plus its rank
+// among the equal-digit lanes (found with 8 ballots), with no barrier between
+// the rounds.  Then the digits' counts are added over waves and digits, the
+// tile's keys and values are put in order in LDS and written from there, so
+// that a digit's run goes out in whole lines.  (Rounds of 256 pairs, four
+// barriers each, written straight from the lanes: 31M 12-byte pairs @@ ms a
+// pass, now @@.)
+template <class K, class V>
+__global__ __launch_bounds__(kRsBlock) void k_rs_scatter(const K* kin, const V* vin, int64_t n,
                                                          int shift, const uint32_t* offs,
-                                                         int ntiles, uint64_t* kout,
-                                                         uint32_t* vout) {
-  __shared__ uint32_t run[kRsBins];
+                                                         int ntiles, K* kout, V* vout) {
   __shared__ uint32_t wc[kRsWaves][kRsBins];
-  const int t = threadIdx.x, w = t / kWave;
-  run[t] = offs[int64_t(t) * ntiles + blockIdx.x];
-  int64_t base = int64_t(blockIdx.x) * kRsTile;
-  for (int r = 0; r < kRsRounds; ++r) {
+  __shared__ uint32_t s_tile[kRsBins], s_run[kRsBins];
+  __shared__ int s_scan[kRsWaves];
+  __shared__ uint8_t s_dig[kRsTile];
+  __shared__ uint64_t s_buf[kRsTile];
+  const int t = threadIdx.x, w = t / kWave, lane = t & (kWave - 1);
+  const int64_t base = int64_t(blockIdx.x) * kRsTile;
+  const int64_t first = base + w * (kRsItems * kWave) + lane;
+  const uint32_t off = offs[int64_t(t) * ntiles + blockIdx.x];
+  K key[kRsItems];
+  V val[kRsItems];
+  uint32_t rank[kRsItems];
 #pragma unroll
-    for (int ww = 0; ww < kRsWaves; ++ww) wc[ww][t] = 0;
-    __syncthreads();
-    int64_t p = base + r * kRsBlock + t;
-    bool valid = p < n;
-    uint64_t key = valid ? kin[p] : 0;
-    uint32_t val = valid ? vin[p] : 0;
-    uint32_t digit = uint32_t(key >> shift) & 0xff;
+  for (int r = 0; r < kRsItems; ++r) {
+    const int64_t p = first + r * kWave;
+    key[r] = p < n ? kin[p] : K(0);
+    val[r] = p < n ? vin[p] : V(0);
+  }
+#pragma unroll
+  for (int ww = 0; ww < kRsWaves; ++ww) wc[ww][t] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kRsItems; ++r) {
+    const bool valid = first + r * kWave < n;
+    const uint32_t digit = uint32_t(key[r] >> shift) & 0xff;
     uint64_t m = __ballot(valid);
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
-      bool bit = (digit >> b) & 1;
-      uint64_t bb = __ballot(bit);
+      const bool bit = (digit >> b) & 1;
+      const uint64_t bb = __ballot(bit);
       m &= bit ? bb : ~bb;
     }
-    uint64_t lower = m & lanemask_lt();
-    if (valid && lower == 0) wc[w][digit] = uint32_t(__popcll(m));
-    __syncthreads();
-    if (valid) {
-      uint32_t dst = run[digit] + uint32_t(__popcll(lower));
-      for (int ww = 0; ww < w; ++ww) dst += wc[ww][digit];
-      kout[dst] = key;
-      vout[dst] = val;
-    }
-    __syncthreads();
-    uint32_t add = 0;
-#pragma unroll
-    for (int ww = 0; ww < kRsWaves; ++ww) add += wc[ww][t];
-    run[t] += add;
-    __syncthreads();
+    const uint32_t before = uint32_t(__popcll(m & lanemask_lt()));
+    const uint32_t had = wc[w][digit];
+    // the wave's LDS accesses keep their order: every lane has read its count
+    asm volatile("" ::: "memory");
+    if (valid && before == 0) wc[w][digit] = had + uint32_t(__popcll(m));
+    asm volatile("" ::: "memory");
+    rank[r] = had + before;
   }
+  __syncthreads();
+  int sum = 0;  // of digit t
+#pragma unroll
+  for (int ww = 0; ww < kRsWaves; ++ww) {
+    const int c = int(wc[ww][t]);
+    wc[ww][t] = uint32_t(sum);
+    sum += c;
+  }
+  int tot;
+  const int pre = block_exclusive_scan<int, kRsBlock>(sum, s_scan, &tot);
+  s_tile[t] = uint32_t(pre);
+  s_run[t] = off - uint32_t(pre);  // + place in the tile = place in the output
+  __syncthreads();
+  K* bk = reinterpret_cast<K*>(s_buf);
+#pragma unroll
+  for (int r = 0; r < kRsItems; ++r) {
+    const uint32_t digit = uint32_t(key[r] >> shift) & 0xff;
+    rank[r] += s_tile[digit] + wc[w][digit];
+    if (first + r * kWave < n) {
+      bk[rank[r]] = key[r];
+      s_dig[rank[r]] = uint8_t(digit);
+    }
+  }
+  __syncthreads();
+  for (int i = t; i < tot; i += kRsBlock) kout[s_run[s_dig[i]] + uint32_t(i)] = bk[i];
+  __syncthreads();
+  V* bv = reinterpret_cast<V*>(s_buf);
+#pragma unroll
+  for (int r = 0; r < kRsItems; ++r)
+    if (first + r * kWave < n) bv[rank[r]] = val[r];
+  __syncthreads();
+  for (int i = t; i < tot; i += kRsBlock) vout[s_run[s_dig[i]] + uint32_t(i)] = bv[i];
 }
 
 struct SortBufs {
@@ -109,26 +148,32 @@ bool take_sort(Carver& c, int64_t n, SortBufs* b) {
   return c.ok;
 }
 
-// Sorts (k[0], v[0]) by bits [0, bits) of the key; returns the buffer index
-// holding the result.
-int radix_sort(SortBufs& b, int64_t n, int bits, hipStream_t st, int* result) {
+// Sorts (k[0], v[0]) by bits [0, bits) of the key; *result: the buffer index
+// holding the sorted pairs.
+template <class K, class V>
+int radix_sort_kv(K* const (&k)[2], V* const (&v)[2], uint32_t* hist, uint32_t* offs,
+                  void* scan_ws, size_t scan_bytes, int64_t n, int bits, hipStream_t st,
+                  int* result) {
   int cur = 0;
   if (n > int64_t(UINT32_MAX)) return fail(RAPTR_ERR_INVALID_ARG, "sort length exceeds 2^32");
   int64_t ntiles = (n + kRsTile - 1) / kRsTile;
   for (int shift = 0; shift < bits; shift += 8) {
-    hipLaunchKernelGGL(k_rs_hist, dim3(unsigned(ntiles)), dim3(kRsBlock), 0, st,
-                       (const uint64_t*)b.k[cur], n, shift, b.hist, int(ntiles));
+    hipLaunchKernelGGL(k_rs_hist<K>, dim3(unsigned(ntiles)), dim3(kRsBlock), 0, st,
+                       (const K*)k[cur], n, shift, hist, int(ntiles));
     RAPTR_LAUNCH_CHECK();
-    RAPTR_TRY(scan_exclusive_u32(b.hist, b.offs, ntiles * kRsBins, nullptr, b.scan_ws,
-                                 b.scan_bytes, st));
-    hipLaunchKernelGGL(k_rs_scatter, dim3(unsigned(ntiles)), dim3(kRsBlock), 0, st,
-                       (const uint64_t*)b.k[cur], (const uint32_t*)b.v[cur], n, shift,
-                       (const uint32_t*)b.offs, int(ntiles), b.k[cur ^ 1], b.v[cur ^ 1]);
+    RAPTR_TRY(scan_exclusive_u32(hist, offs, ntiles * kRsBins, nullptr, scan_ws, scan_bytes, st));
+    hipLaunchKernelGGL((k_rs_scatter<K, V>), dim3(unsigned(ntiles)), dim3(kRsBlock), 0, st,
+                       (const K*)k[cur], (const V*)v[cur], n, shift, (const uint32_t*)offs,
+                       int(ntiles), k[cur ^ 1], v[cur ^ 1]);
     RAPTR_LAUNCH_CHECK();
     cur ^= 1;
   }
   *result = cur;
   return RAPTR_OK;
+}
+int radix_sort(SortBufs& b, int64_t n, int bits, hipStream_t st, int* result) {
+  return radix_sort_kv<uint64_t, uint32_t>(b.k, b.v, b.hist, b.offs, b.scan_ws, b.scan_bytes, n,
+                                           bits, st, result);
 }
 
 int bits_for(uint64_t maxval) {
@@ -278,6 +323,33 @@ int radix_sort_pairs(uint64_t* k0, uint64_t* k1, uint32_t* v0, uint32_t* v1, int
   if (!cv.ok) return fail(RAPTR_ERR_WORKSPACE, "radix sort scratch too small");
   return radix_sort(b, n, bits, st, result);
 }
+
+size_t sort_scratch_bytes(int64_t n) {
+  const int64_t ntiles = (n + kRsTile - 1) / kRsTile;
+  Sizer z;
+  z.take<uint32_t>(size_t(ntiles * kRsBins));
+  z.take<uint32_t>(size_t(ntiles * kRsBins));
+  z.take<char>(scan_workspace_bytes(ntiles * kRsBins));
+  return z.bytes() + 512;
+}
+
+template <class K>
+int radix_sort_payload(K* k0, K* k1, uint64_t* v0, uint64_t* v1, int64_t n, int bits,
+                       hipStream_t st, int* result, Carver& cv) {
+  const int64_t ntiles = (n + kRsTile - 1) / kRsTile;
+  uint32_t* hist = cv.take<uint32_t>(size_t(ntiles * kRsBins));
+  uint32_t* offs = cv.take<uint32_t>(size_t(ntiles * kRsBins));
+  const size_t sb = scan_workspace_bytes(ntiles * kRsBins);
+  void* sw = cv.take<char>(sb);
+  if (!cv.ok) return fail(RAPTR_ERR_WORKSPACE, "radix sort scratch too small");
+  K* const k[2] = {k0, k1};
+  uint64_t* const v[2] = {v0, v1};
+  return radix_sort_kv<K, uint64_t>(k, v, hist, offs, sw, sb, n, bits, st, result);
+}
+template int radix_sort_payload<uint32_t>(uint32_t*, uint32_t*, uint64_t*, uint64_t*, int64_t, int,
+                                          hipStream_t, int*, Carver&);
+template int radix_sort_payload<uint64_t>(uint64_t*, uint64_t*, uint64_t*, uint64_t*, int64_t, int,
+                                          hipStream_t, int*, Carver&);
 
 }  // namespace raptr
 
