@@ -1713,8 +1713,9 @@ __global__ __launch_bounds__(64 * W) void k_fb1l(int64_t m, int rows,
 // x'_j = x_j c_j / (s_j + (s_j == 0)) and an FP64 partial sum per
 // workgroup.  Workgroups of one XCD take consecutive columns, whose
 // partials lie side by side in each group's sorted union; each takes `per`
-// runs of 256 / LPC of them, so that at most about 2,048 partial sums are left
-// for k_norm_scale.
+// runs of 256 / LPC of them, so that at most 16,384 partial sums are left for
+// k_norm_scale (one run each up to 262,144 columns at LPC = 16: five runs in
+// turn took 57 us at 52^3, one 30).
 template <int LPC, int U>
 __global__ __launch_bounds__(256) void k_fb1_reduce(int n, int per,
                                                     const int64_t* __restrict__ vptr,
@@ -2282,9 +2283,9 @@ __global__ __launch_bounds__(256) void k_norms(const double* partials, int nb, i
 // One frame: k_norms and k_scale_frames in one launch.  Every workgroup adds
 // the partial sums itself, in k_norms' order (the same bits), then scales its
 // share of x'.  Two launches of 3 us each and the gap between them less, of 39
-// us per iteration at 32^3; up to kNormScaleMax partial sums (32 KiB from L2
-// per workgroup), where they take longer than a launch.
-constexpr int kNormScaleMax = 4096;
+// us per iteration at 32^3; up to kNormScaleMax partial sums (128 KiB from L2
+// per workgroup: 8,788 of them 12 us, 2,048 5.4).
+constexpr int kNormScaleMax = 16384;
 __global__ __launch_bounds__(256) void k_norm_scale(const double* __restrict__ partials, int nb,
                                                     int64_t n, const float* __restrict__ xx,
                                                     float* scale, double* norm,
@@ -2853,7 +2854,7 @@ int launch_fused1(const raptr_recon* R, const float* x, const float* y, hipStrea
     return RAPTR_OK;
   }
   const int64_t runs = (int64_t(n) + (256 / L) - 1) / (256 / L);
-  const int per = int((runs + 2047) / 2048);
+  const int per = int((runs + 16383) / 16384);
   const unsigned nr = unsigned((runs + per - 1) / per);
 #define RAPTR_FR(LL)                                                                           \
   if (L == LL)                                                                                 \

@@ -76,10 +76,10 @@ def test_mode1_reduce_both_forms(gpu, grid, split):
     assert _rel(images[0], images[1]) <= 1e-6
 
 
-@pytest.mark.parametrize("grid", [VoxelGrid((-50.0, -50.0, -50.0), (1.0, 1.0, 1.0), (104, 101, 103)),
+@pytest.mark.parametrize("grid", [VoxelGrid((-66.0, -64.4, -65.2), (0.8, 0.8, 0.8), (165, 161, 163)),
                                   centred_grid(17, 5.0)], ids=["2 launches", "1 launch"])
 def test_normalisation_launches(gpu, grid):
-    """More than 4,096 partial sums (1.08M voxels) and fewer."""
+    """More than 16,384 partial sums (4.33M voxels) and fewer."""
     from raptr_amd.recon import Reconstructor
     setup = two_head_setup(6, 5, 36.0)
     A, dsens, sens, mat, y = _system(setup, grid, 6, rows=700)
