@@ -77,7 +77,10 @@ struct Pool {
   std::unordered_map<void*, PoolBlock> live;  // blocks handed out
   std::list<PoolBlock> kept;                  // oldest first
   std::map<int, size_t> kept_bytes;
-  std::map<int, hipStream_t> clear;           // the stream that clears, per device
+  // recorded after the last clearing, per device.  Blocks are cleared on the null
+  // stream: a stream of the pool's own would take one of the process's hardware
+  // queues and make two of a caller's streams share another
+  std::map<int, hipEvent_t> cleared;
 };
 // never destroyed: frees may come while the process ends
 Pool& pool() {
@@ -112,7 +115,7 @@ hipError_t pool_malloc(void** p, size_t bytes) {
           (best == P.kept.end() || it->bytes < best->bytes))
         best = it;
     // (its clearing, asked for when it was freed, has mostly long ended)
-    if (best != P.kept.end() && hipStreamSynchronize(P.clear[dev]) == hipSuccess) {
+    if (best != P.kept.end() && hipEventSynchronize(P.cleared[dev]) == hipSuccess) {
       *p = best->p;
       P.live[best->p] = *best;
       P.kept_bytes[dev] -= best->bytes;
@@ -161,9 +164,10 @@ hipError_t pool_free(void* p, bool idle) {
     return hipFree(p);
   }
   std::lock_guard<std::mutex> lock(P.mu);
-  hipStream_t& st = P.clear[dev];
-  if ((!st && hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess) ||
-      hipMemsetAsync(b.p, 0, b.bytes, st) != hipSuccess) {
+  hipEvent_t& ev = P.cleared[dev];
+  if ((!ev && hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) ||
+      hipMemsetAsync(b.p, 0, b.bytes, nullptr) != hipSuccess ||
+      hipEventRecord(ev, nullptr) != hipSuccess) {
     (void)hipGetLastError();
     return hipFree(p);
   }
