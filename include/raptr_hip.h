@@ -614,8 +614,9 @@ int raptr_recon_get_broadcast(const raptr_recon* plan);
  * keys and values from coalesced vector loads; the backward adds each
  * launch's row blocks into one shared image sum), kind 3 (the default) =
  * kind 2 with a backward in which each XCD takes one eighth of the row
- * blocks and writes its own partial image (8 x n x 64 floats, allocated
- * with the plan); a fixed-order reduce adds them.  Shapes per G: 16: unroll
+ * blocks (a quarter, half or all of them on plans of few rows) and writes
+ * its range's partial image (8 x n x 64 floats, allocated with the plan); a
+ * fixed-order reduce adds them.  Shapes per G: 16: unroll
  * 8, 16 or 32, kind 2 or 3; 32: unroll 8 or 16, kind 3
  * (v_mfma_f32_32x32x2f32, 2 entries x 32 frames, whole 128-byte lines per
  * gathered frame block).  Voxel bricks: 4x1x4 (G = 16), 4x2x4 (G = 32).

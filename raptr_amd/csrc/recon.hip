@@ -1281,7 +1281,8 @@ __global__ __launch_bounds__(256) void k_bwdm64(int ngc, const int64_t* __restri
 
 // Backward with per-XCD row ranges (64 frames, bricks of G = 16 or 32):
 // workgroup i runs on XCD i % 8 (the dispatcher's round-robin), which takes
-// row blocks [nblk*x/8, nblk*(x+1)/8).  Each wave walks its brick through
+// row blocks [nblk*x/8, nblk*(x+1)/8) (nr < 8 ranges, backward_ranges: 8 / nr
+// XCDs share a range and split its bricks).  Each wave walks its brick through
 // all of its XCD's blocks; the bricks resident on one XCD at a time are
 // consecutive (neighbouring voxels) and walk the same small ratio slices
 // together, so their ratio gathers hit that XCD's L2.  Each XCD writes its
@@ -1302,16 +1303,16 @@ __global__ __launch_bounds__(256) void k_bwdm64x(int ngc, int nblk, int n,
                                                  const typename Val<VT>::T* __restrict__ gval,
                                                  const int* __restrict__ cols,
                                                  const float* __restrict__ e,
-                                                 float* __restrict__ c8, int boff, int bcnt,
-                                                 int accum) {
+                                                 float* __restrict__ c8, int nr, int boff,
+                                                 int bcnt, int accum) {
   using M = MF<G>;
   constexpr int U = 8 / M::K;  // 8-entry steps (backward lists are aligned to 8)
   const int lane = threadIdx.x & (kWave - 1);
   const int kq = lane / M::W, rw = lane % M::W;
-  const int xcd = int(blockIdx.x % 8);
-  const int h = int(blockIdx.x / 8) * (256 / kWave) + wave_id();
+  const int xcd = int(blockIdx.x % 8) * nr / 8, sub = int(blockIdx.x % 8) % (8 / nr);
+  const int h = (int(blockIdx.x / 8) * (8 / nr) + sub) * (256 / kWave) + wave_id();
   if (h >= ngc) return;
-  const int b0 = int(int64_t(nblk) * xcd / 8), b1 = int(int64_t(nblk) * (xcd + 1) / 8);
+  const int b0 = int(int64_t(nblk) * xcd / nr), b1 = int(int64_t(nblk) * (xcd + 1) / nr);
   const int s0 = b0 + boff < b1 ? b0 + boff : b1;
   const int s1 = s0 + bcnt < b1 ? s0 + bcnt : b1;
   typename M::acc_t acc[FB];
@@ -1332,13 +1333,13 @@ __global__ __launch_bounds__(256) void k_bwdm64x(int ngc, int nblk, int n,
   }
 }
 
-// c = sum of the 8 partial images (XCD order), x' = x*c/(s + (s==0)), and
+// c = sum of the nr partial images (range order), x' = x*c/(s + (s==0)), and
 // FP64 partial sums per workgroup (4 * per voxels) and frame; frames fa .. 63
 // are skipped (x' and their partial sums not written).  per: voxels in turn,
 // so that some 2,048 rows of partial sums are left for k_norms (one row per
 // 4 voxels made 18 MB of them at 52^3: 62 us here and 67 there,
 // now 45 and 13).
-__global__ __launch_bounds__(256) void k_bwd_xreduce(int n, int fa, int per,
+__global__ __launch_bounds__(256) void k_bwd_xreduce(int n, int fa, int nr, int per,
                                                      const float* __restrict__ c8,
                                                      const float* __restrict__ x,
                                                      const float* __restrict__ s,
@@ -1351,9 +1352,8 @@ __global__ __launch_bounds__(256) void k_bwd_xreduce(int n, int fa, int per,
     for (int it = 0; it < per; ++it) {
       const int64_t j = (int64_t(blockIdx.x) * per + it) * 4 + jj;
       if (j >= n) break;
-      float cv = 0.0f;
-#pragma unroll
-      for (int q = 0; q < 8; ++q) cv += c8[(int64_t(q) * n + j) * 64 + f];
+      float cv = c8[j * 64 + f];
+      for (int q = 1; q < nr; ++q) cv += c8[(int64_t(q) * n + j) * 64 + f];
       float d = s[j];
       d += float(d == 0.0f);
       const float nv = x[j * 64 + f] * cv / d;
@@ -2681,13 +2681,39 @@ int launch_bwd1_xcd(const raptr_recon* R, const float* x, hipStream_t st, int* n
   return RAPTR_OK;
 }
 
+// Row ranges (8, 4, 2 or 1) of the kind-3 backward.  Each writes a partial
+// image, read once more by k_bwd_xreduce (0.155 us per 1,000 voxels and range,
+// measured at 96^3), and the fewer they are the more ratio rows an XCD gathers
+// from: 33 us per 1M union entries with 8, 1.15, 1.6 and 2.4 times that with 4,
+// 2 and 1.  Fewer than 8 only where 32,768 waves are left.  Backward with 8, 4,
+// 2, 1 ranges: 20,249 rows at 96^3 1,258, 708, 435, 338 us; 98,454 rows 1,552,
+// 952, 748, 807; 286,441 rows 2,227, 1,569, 1,632, 2,187; 39,730 rows at 52^3
+// 282, 163, 171, 240; 147,579 rows 480, 408, 543; 379,499 rows 933, 972, 1,424;
+// 20,282 rows at 32^3 (2,048 bricks) 110, 133, 133.
+int backward_ranges(int64_t entries, int n, int64_t bricks) {
+  const double factor[4] = {1.0, 1.15, 1.6, 2.4};
+  int best = 8;
+  double least = 1e300;
+  for (int k = 0, nr = 8; k < 4; ++k, nr /= 2) {
+    if (nr < 8 && bricks * nr < 32768) break;
+    const double us = 0.155e-3 * double(n) * nr + 33e-6 * double(entries) * factor[k];
+    if (us < least) {
+      least = us;
+      best = nr;
+    }
+  }
+  return best;
+}
+
 // 64-frame backward with per-XCD row ranges and partial images, then the
 // reduce + update (grouped layouts of 16, kind 3)
 int launch_bwd_xcd(const raptr_recon* R, const float* x, hipStream_t st, int* nb_out) {
   if (!R->c8 || R->grp_g < 16)
     return fail(RAPTR_ERR_INVALID_ARG, "plan has no per-XCD partial images");
-  const unsigned gg = unsigned(8 * ((R->ngc + 3) / 4));
-  const int per_xcd = (R->nblk + 7) / 8;  // most blocks of any XCD's range
+  const int nrg = R->grp_ranges;
+  const int64_t wgs = (R->ngc + 3) / 4;
+  const unsigned gg = unsigned(8 * ((wgs * nrg + 7) / 8));
+  const int per_xcd = (R->nblk + nrg - 1) / nrg;  // most blocks of any range
   const int bpl = R->xcd_bpl > 0 ? R->xcd_bpl : per_xcd;
   const int FBA = R->fa / R->grp_g;
   for (int boff = 0; boff < per_xcd; boff += bpl) {
@@ -2698,7 +2724,7 @@ int launch_bwd_xcd(const raptr_recon* R, const float* x, hipStream_t st, int* nb
     hipLaunchKernelGGL((k_bwdm64x<VV, G_, FB_>), dim3(gg), dim3(256), 0, st, int(R->ngc),     \
                        R->nblk, R->n, (const int64_t*)R->gbp, (const int*)R->gbrow,          \
                        (const typename Val<VV>::T*)R->gbval, (const int*)R->gcols,           \
-                       (const float*)R->e, R->c8, boff, bpl, accum);                         \
+                       (const float*)R->e, R->c8, nrg, boff, bpl, accum);                    \
     launched = true;                                                                         \
   }
 #define RAPTR_X64V(VV)                                                                       \
@@ -2712,7 +2738,7 @@ int launch_bwd_xcd(const raptr_recon* R, const float* x, hipStream_t st, int* nb
   const int64_t quads = (int64_t(R->n) + 3) / 4;
   const int per = int((quads + 2047) / 2048);
   const unsigned nr = unsigned((quads + per - 1) / per);
-  hipLaunchKernelGGL(k_bwd_xreduce, dim3(nr), dim3(256), 0, st, R->n, R->fa, per,
+  hipLaunchKernelGGL(k_bwd_xreduce, dim3(nr), dim3(256), 0, st, R->n, R->fa, nrg, per,
                      (const float*)R->c8, x, (const float*)R->s, R->xx, R->partials);
   RAPTR_LAUNCH_CHECK();
   if (nb_out) *nb_out = int(nr);
@@ -3749,8 +3775,9 @@ int create_plan(raptr_recon** out, int m, int n, int64_t nnz, const int64_t* d_r
 #undef RAPTR_CG
           }
         }
-        // per-XCD partial images of the kind-3 backward
-        if (!rc) rc = ralloc(R, &R->c8, size_t(8) * n * 64);
+        // partial images of the kind-3 backward
+        R->grp_ranges = backward_ranges(R->gbnnz, n, R->ngc);
+        if (!rc) rc = ralloc(R, &R->c8, size_t(R->grp_ranges) * n * 64);
         if (!rc) R->grp64 = 1;
       }
       (void)hipStreamSynchronize(st);

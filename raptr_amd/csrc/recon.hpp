@@ -134,6 +134,7 @@ struct raptr_recon {
   int grp64 = 0;       // use the grouped kernels for 64-frame passes
   int grp_g = 16;      // members per group (16, 32)
   int* gcols = nullptr;  // ngc * grp_g member columns of the backward groups (-1: none)
+  int grp_ranges = 8;  // row ranges of the kind-3 backward
   int grp_unroll = 8;  // union entries in flight per wave (4, 8, 16)
   int grp_pipe = 1;    // kernel kind: 0 plain, 1 pipelined scalar loads, 2 matrix cores,
                        // 3 matrix cores with per-XCD row ranges in the backward

@@ -141,3 +141,28 @@ def test_frames64_both_forwards(gpu, rows, grid, vt):
     for f in (0, 1, 31, 62):
         assert _rel(X[:, f], R1.mlem(np.ascontiguousarray(Y[:, f]), _x0(grid.nvox), 4)) <= 1e-6
     assert np.all(X[:, 63] == 0.0)
+
+
+@pytest.mark.parametrize("n", [(64, 48, 49), (72, 66, 64), (96, 97, 64)])
+def test_frames64_few_ranges(gpu, n):
+    """Grids of 9,408, 19,008 and 37,248 bricks under few rows: the backward
+    splits its rows in 4, 2 and 1 ranges.  The first 16 frames alone get the
+    full pass's images."""
+    from raptr_amd.device import DeviceArray
+    from raptr_amd.recon import Reconstructor
+    setup = two_head_setup(6, 8, 22.5)
+    grid = VoxelGrid(tuple(-0.5 * k for k in n), (1.0, 1.0, 1.0), n)
+    A, dsens, _, _, y = _system(setup, grid, 5, rows=601)
+    R = Reconstructor(A, dsens, "f32", 64, row_order=setup, grid=grid)
+    Y = np.repeat(y[:, None], 64, axis=1)
+    Y[:, 1:] *= np.random.default_rng(6).integers(1, 4, (A.m, 63)).astype(np.float32)
+    X0 = np.repeat(_x0(grid.nvox)[:, None], 64, axis=1)
+    X = R.mlem(Y, X0, 4)
+    dy, dx = DeviceArray.from_numpy(Y.reshape(-1)), DeviceArray.from_numpy(X0.reshape(-1))
+    R.run(dy, dx, 4, 64, use_graph=False, active=16)
+    np.testing.assert_array_equal(dx.numpy().reshape(grid.nvox, 64)[:, :16], X[:, :16])
+    R.close()
+    R1 = Reconstructor(A, dsens, "f32", 1, row_order=setup)
+    for f in (0, 15, 40, 63):
+        want = R1.mlem(np.ascontiguousarray(Y[:, f]), _x0(grid.nvox), 4)
+        assert _rel(X[:, f], want) <= 1e-6
