@@ -19,6 +19,7 @@
 //         dropped with a second ballot compaction into an LDS row buffer;
 //      4. row buffers are flushed as pieces into a staging area and packed
 //         into a CSR with 64-bit row pointers per channel chunk.
+#include <atomic>
 #include <cmath>
 #include <mutex>
 
@@ -1201,13 +1202,21 @@ size_t rays_lds_bytes(const BuildArgs& A) {
               (lists > rays ? lists : rays));
 }
 
-template <class K>
-int launch_rows(K kernel, const BuildArgs& A, size_t lds, hipStream_t st, int threads = kSmBlock) {
-  // Raise the dynamic-LDS limit; not fatal where the default suffices.
-  if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          160 * 1024) != hipSuccess)
-    (void)hipGetLastError();
-  hipLaunchKernelGGL(kernel, dim3(unsigned(A.rows)), dim3(threads), lds, st, A);
+template <void (*KERNEL)(BuildArgs)>
+int launch_rows(const BuildArgs& A, size_t lds, hipStream_t st, int threads = kSmBlock) {
+  // the kernel's dynamic-LDS limit raised on its first launch per device; not
+  // fatal where the default suffices
+  static std::atomic<uint64_t> raised{0};
+  int dev = 0;
+  RAPTR_HIP_TRY(hipGetDevice(&dev));
+  const uint64_t bit = uint64_t(1) << (dev & 63);
+  if (!(raised.load() & bit)) {
+    if (hipFuncSetAttribute((const void*)KERNEL, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            160 * 1024) != hipSuccess)
+      (void)hipGetLastError();
+    raised.fetch_or(bit);
+  }
+  hipLaunchKernelGGL(KERNEL, dim3(unsigned(A.rows)), dim3(threads), lds, st, A);
   RAPTR_LAUNCH_CHECK();
   return RAPTR_OK;
 }
@@ -1221,14 +1230,14 @@ int launch_build(const BuildArgs& A, size_t lds, hipStream_t st) {
   const size_t lr = rays_lds_bytes(A);
   if (A.by_candidate || A.raygen == RAPTR_RAYGEN_RAND_ELEMENT || A.keep_zeros || lr > 156 * 1024 ||
       int64_t(A.G.g.n[0]) * A.G.g.n[1] >= 1 << 24)
-    return launch_rows(k_sm_build<MODE>, A, lds, st);
+    return launch_rows<k_sm_build<MODE>>(A, lds, st);
   // Two waves a row where the rays' tables are small, four else: a wave's
   // share of each phase must outlast the barriers.  147,456 rows of 10 rays x
   // 99 planes: 0.96 ms with two, 1.02 with four; 40,009 of 17 x 131: 1.04 and
   // 0.98; 100,003 of 30 x 159: 2.23 and 1.78 (8 waves: 2.24).
-  if (A.rpb > 1) return launch_rows(k_sm_rays<MODE, false, 4>, A, lr, st, 256);
-  if (A.nrays * A.pl < 1536) return launch_rows(k_sm_rays<MODE, true, 2>, A, lr, st, 128);
-  return launch_rows(k_sm_rays<MODE, true, 4>, A, lr, st, 256);
+  if (A.rpb > 1) return launch_rows<k_sm_rays<MODE, false, 4>>(A, lr, st, 256);
+  if (A.nrays * A.pl < 1536) return launch_rows<k_sm_rays<MODE, true, 2>>(A, lr, st, 128);
+  return launch_rows<k_sm_rays<MODE, true, 4>>(A, lr, st, 256);
 }
 
 // Workspace layout of the fused build for a staging area of S entries:
