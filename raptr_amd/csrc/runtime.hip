@@ -58,9 +58,9 @@ int make_geom(const raptr_setup_t* setup, const raptr_grid_t* grid, Geom* G) {
 // Cache of freed device blocks.  A reconstruction of 30M entries allocates and
 // frees 2.2 GB in 60 blocks: 8 ms of a 19 ms call in the driver, and 85 ms once
 // the device's cleared memory is used up, since the driver clears a freed block
-// before it hands it out again (some 26 GB/s).  Freed blocks of up to kPoolBlock
+// before it hands it out again.  Freed blocks of up to kPoolBlock
 // bytes are kept, up to kPoolBytes per device, the oldest given back first, all
-// of them when an allocation finds no memory.  A kept block is cleared at 4 TB/s
+// of them when an allocation finds no memory.  A kept block is cleared
 // when it is freed, so a caller sees what it saw before: idle, cleared memory.
 // Sizes are rounded to eighths of a power of two, so that lists of similar
 // length find each other's blocks.

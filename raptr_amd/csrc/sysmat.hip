@@ -2,11 +2,15 @@
 //
 // Two entry points follow the reference:
 //  * raptr_sm_from_wq: the two-stage path (getSystemMatrixFromWorkqueue.cu:
-//    116-281), one thread per workqueue entry, rays of the entry's channel
-//    regenerated from the counter-based Philox stream.
+//    116-281): queues in channel order by runs of a channel, its rays and
+//    plane tables made once (k_sm_from_wq_runs); other entries by rays made
+//    anew from the counter-based Philox stream.
 //  * raptr_sm_build_csr: the production path (what getSystemMatrix +
 //    cooSort + coo2csr + csr2ecsr produce, getSystemMatrixDeviceOnly.cu:
-//    357-562, wrappers.hpp:185-266), one workgroup per channel:
+//    357-562, wrappers.hpp:185-266), one workgroup per channel.
+//    k_sm_rays (see there) marks the voxels that each ray can meet and samples
+//    only those; k_sm_build serves what it does not take (per-element rays,
+//    zeros kept, masks larger than the LDS), with the steps:
 //      1. the channel's rays are generated once into LDS, with per-ray plane
 //         tables alpha[dim][k] = (o + k*d - r0)/(r1 - r0) for every grid plane
 //         (the voxel-box divisions of the slab method depend only on the
