@@ -113,15 +113,19 @@ def build_cpp_io_test():
 
 
 CPP_TESTS = [os.path.join(ROOT, "tests", "cpp", "test_reference_api.cpp")]
+# host-only programs over headers of csrc/, without the library
+CPP_UNIT_TESTS = [os.path.join(ROOT, "tests", "cpp", "test_block_cache.cpp")]
 
 
 def build_cpp_tests():
     """C++ programs written against include/raptr/*.hpp, linked to the HIP
-    library (rpath to raptr_amd/lib)."""
-    for src in CPP_TESTS:
+    library (rpath to raptr_amd/lib), and the host-only ones."""
+    link = [f"-L{LIBDIR}", "-lraptr_hip", "-Wl,-rpath,$ORIGIN"]
+    for src, flags in [(s, link) for s in CPP_TESTS] + [(s, [f"-I{CSRC}"])
+                                                       for s in CPP_UNIT_TESTS]:
         out = os.path.join(LIBDIR, os.path.basename(src)[:-4])
         cmd = ["g++", "-O2", "-std=c++17", "-Wall", f"-I{os.path.join(ROOT, 'include')}", src,
-               "-o", out + ".tmp", f"-L{LIBDIR}", "-lraptr_hip", "-Wl,-rpath,$ORIGIN"]
+               "-o", out + ".tmp"] + flags
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError(f"g++ failed for {src}:\n{r.stdout}\n{r.stderr}")

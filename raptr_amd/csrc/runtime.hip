@@ -1,14 +1,11 @@
 // runtime.hip -- status/error plumbing, device memory and stream helpers,
 // host-side geometry tables.
-#include <list>
-#include <map>
-#include <mutex>
-#include <unordered_map>
-
 #include <cmath>
 #include <cstdarg>
 #include <cstring>
+#include <map>
 
+#include "blockcache.hpp"
 #include "common.hpp"
 
 namespace raptr {
@@ -55,142 +52,48 @@ int make_geom(const raptr_setup_t* setup, const raptr_grid_t* grid, Geom* G) {
   return RAPTR_OK;
 }
 
-// Cache of freed device blocks.  A reconstruction of 30M entries allocates and
-// frees 2.2 GB in 60 blocks: 8 ms of a 19 ms call in the driver, and 85 ms once
-// the device's cleared memory is used up, since the driver clears a freed block
-// before it hands it out again.  Freed blocks of up to kPoolBlock
-// bytes are kept, up to kPoolBytes per device, the oldest given back first, all
-// of them when an allocation finds no memory.  A kept block is cleared
-// when it is freed, so a caller sees what it saw before: idle, cleared memory.
-// Sizes are rounded to eighths of a power of two, so that lists of similar
-// length find each other's blocks.
+// Device memory through the block cache (blockcache.hpp).
 namespace {
-constexpr size_t kPoolBlock = size_t(1) << 30;
-constexpr size_t kPoolBytes = size_t(4) << 30;
-struct PoolBlock {
-  void* p;
-  size_t bytes;
-  int dev;
-};
-struct Pool {
-  std::mutex mu;
-  std::unordered_map<void*, PoolBlock> live;  // blocks handed out
-  std::list<PoolBlock> kept;                  // oldest first
-  std::map<int, size_t> kept_bytes;
+struct HipDriver {
+  using Error = hipError_t;
+  static constexpr hipError_t kOk = hipSuccess, kNoMemory = hipErrorOutOfMemory,
+                              kInvalid = hipErrorInvalidValue;
+  hipError_t device(int* dev) { return hipGetDevice(dev); }
+  hipError_t alloc(void** p, size_t bytes) { return hipMalloc(p, bytes); }
+  hipError_t release(void* p) { return hipFree(p); }
+  size_t extent(void* p) {
+    hipDeviceptr_t base = nullptr;
+    size_t bytes = 0;
+    if (hipMemGetAddressRange(&base, &bytes, p) == hipSuccess && base == p) return bytes;
+    (void)hipGetLastError();
+    return 0;
+  }
+  hipError_t wait() { return hipDeviceSynchronize(); }
+  hipError_t clear(void* p, size_t bytes, int dev) {
+    hipEvent_t& ev = cleared[dev];
+    if (!ev) {
+      const hipError_t e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+      if (e != hipSuccess) return e;
+    }
+    const hipError_t e = hipMemsetAsync(p, 0, bytes, nullptr);
+    return e == hipSuccess ? hipEventRecord(ev, nullptr) : e;
+  }
+  hipError_t wait_clear(int dev) { return hipEventSynchronize(cleared[dev]); }
+  void forget_error() { (void)hipGetLastError(); }
   // recorded after the last clearing, per device.  Blocks are cleared on the null
-  // stream: a stream of the pool's own would take one of the process's hardware
+  // stream: a stream of the cache's own would take one of the process's hardware
   // queues and make two of a caller's streams share another
   std::map<int, hipEvent_t> cleared;
 };
 // never destroyed: frees may come while the process ends
-Pool& pool() {
-  static Pool* p = new Pool;
-  return *p;
-}
-
-size_t pool_size(size_t bytes) {
-  if (bytes <= 4096) return 4096;
-  size_t step = 512;
-  while (step * 16 < bytes) step *= 2;  // bytes in (8, 16] steps
-  return (bytes + step - 1) / step * step;
+BlockCache<HipDriver>& cache() {
+  static BlockCache<HipDriver>* c = new BlockCache<HipDriver>;
+  return *c;
 }
 }  // namespace
 
-hipError_t pool_malloc(void** p, size_t bytes) {
-  *p = nullptr;
-  if (bytes > kPoolBlock) {
-    hipError_t e = hipMalloc(p, bytes);
-    if (e != hipErrorOutOfMemory) return e;
-  }
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
-  const size_t need = bytes > kPoolBlock ? bytes : pool_size(bytes);
-  Pool& P = pool();
-  std::lock_guard<std::mutex> lock(P.mu);
-  if (bytes <= kPoolBlock) {
-    auto best = P.kept.end();
-    for (auto it = P.kept.begin(); it != P.kept.end(); ++it)
-      if (it->dev == dev && it->bytes >= need && it->bytes <= need + need / 4 &&
-          (best == P.kept.end() || it->bytes < best->bytes))
-        best = it;
-    // (its clearing, asked for when it was freed, has mostly long ended)
-    if (best != P.kept.end() && hipEventSynchronize(P.cleared[dev]) == hipSuccess) {
-      *p = best->p;
-      P.live[best->p] = *best;
-      P.kept_bytes[dev] -= best->bytes;
-      P.kept.erase(best);
-      return hipSuccess;
-    }
-    (void)hipGetLastError();
-    e = hipMalloc(p, need);
-  } else {
-    e = hipErrorOutOfMemory;
-  }
-  if (e == hipErrorOutOfMemory && P.kept_bytes[dev]) {
-    (void)hipGetLastError();
-    for (auto it = P.kept.begin(); it != P.kept.end();)
-      if (it->dev == dev) {
-        (void)hipFree(it->p);
-        it = P.kept.erase(it);
-      } else {
-        ++it;
-      }
-    P.kept_bytes[dev] = 0;
-    e = hipMalloc(p, need);
-  }
-  if (e == hipSuccess && bytes <= kPoolBlock) P.live[*p] = PoolBlock{*p, need, dev};
-  return e;
-}
-
-hipError_t pool_free(void* p, bool idle) {
-  if (!p) return hipSuccess;
-  Pool& P = pool();
-  PoolBlock b{nullptr, 0, 0};
-  {
-    std::lock_guard<std::mutex> lock(P.mu);
-    auto it = P.live.find(p);
-    if (it != P.live.end()) {
-      b = it->second;
-      P.live.erase(it);
-    }
-  }
-  int dev = 0;
-  // not the pool's, another device's, or a device that cannot be waited for
-  // (a capture): the driver's own free
-  if (!b.p || hipGetDevice(&dev) != hipSuccess || dev != b.dev ||
-      (!idle && hipDeviceSynchronize() != hipSuccess)) {
-    (void)hipGetLastError();
-    return hipFree(p);
-  }
-  std::lock_guard<std::mutex> lock(P.mu);
-  hipEvent_t& ev = P.cleared[dev];
-  if ((!ev && hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) ||
-      hipMemsetAsync(b.p, 0, b.bytes, nullptr) != hipSuccess ||
-      hipEventRecord(ev, nullptr) != hipSuccess) {
-    (void)hipGetLastError();
-    return hipFree(p);
-  }
-  P.kept.push_back(b);
-  P.kept_bytes[dev] += b.bytes;
-  for (auto it = P.kept.begin(); P.kept_bytes[dev] > kPoolBytes && it != P.kept.end();)
-    if (it->dev == dev) {
-      P.kept_bytes[dev] -= it->bytes;
-      (void)hipFree(it->p);
-      it = P.kept.erase(it);
-    } else {
-      ++it;
-    }
-  return hipSuccess;
-}
-
-static size_t pool_kept_bytes() {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 0;
-  Pool& P = pool();
-  std::lock_guard<std::mutex> lock(P.mu);
-  return P.kept_bytes[dev];
-}
+hipError_t pool_malloc(void** p, size_t bytes) { return cache().malloc(p, bytes); }
+hipError_t pool_free(void* p, bool idle) { return cache().free(p, idle); }
 
 }  // namespace raptr
 
@@ -341,7 +244,7 @@ int raptr_event_elapsed_ms(float* ms, void* a, void* b) {
 }
 int raptr_mem_info(size_t* free_bytes, size_t* total_bytes) {
   RAPTR_HIP_TRY(hipMemGetInfo(free_bytes, total_bytes));
-  if (free_bytes) *free_bytes += pool_kept_bytes();  // given back when needed
+  if (free_bytes) *free_bytes += cache().kept_bytes();  // given back when needed
   return RAPTR_OK;
 }
 

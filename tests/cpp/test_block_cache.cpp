@@ -1,0 +1,179 @@
+// The block cache's rules (raptr_amd/csrc/blockcache.hpp) over a model of the
+// driver: what is handed out is always the driver's, large enough, of the right
+// device, cleared and handed out once.
+#include <cstdint>
+#include <cstdio>
+#include <map>
+#include <set>
+#include <vector>
+
+#include "blockcache.hpp"
+
+static int failures = 0;
+#define CHECK(c)                                                      \
+  do {                                                                \
+    if (!(c)) {                                                       \
+      std::printf("%s:%d: %s\n", __FILE__, __LINE__, #c);             \
+      ++failures;                                                     \
+    }                                                                 \
+  } while (0)
+
+struct Model {
+  enum Error { kOk, kNoMemory, kInvalid, kNoWait };
+  struct Mem {
+    size_t bytes;
+    int dev;
+    bool cleared;
+  };
+  std::map<uintptr_t, Mem> mem;
+  uintptr_t next = 0x1000;
+  size_t used = 0, room = size_t(64) << 30;
+  int dev = 0, allocs = 0, releases = 0, waits = 0, clears = 0;
+  bool can_wait = true;
+  Error device(int* d) {
+    *d = dev;
+    return kOk;
+  }
+  Error place(uintptr_t at, size_t bytes) {
+    mem[at] = Mem{bytes, dev, true};
+    used += bytes;
+    return kOk;
+  }
+  Error alloc(void** p, size_t bytes) {
+    if (used + bytes > room) return kNoMemory;
+    ++allocs;
+    *p = reinterpret_cast<void*>(next);
+    place(next, bytes);
+    next += (bytes + 0xfff) / 0x1000 * 0x1000;
+    return kOk;
+  }
+  Error release(void* p) {
+    auto it = mem.find(uintptr_t(p));
+    if (it == mem.end()) return kInvalid;
+    ++releases;
+    used -= it->second.bytes;
+    mem.erase(it);
+    return kOk;
+  }
+  size_t extent(void* p) {
+    auto it = mem.find(uintptr_t(p));
+    return it == mem.end() ? 0 : it->second.bytes;
+  }
+  Error wait() {
+    ++waits;
+    return can_wait ? kOk : kNoWait;
+  }
+  Error clear(void* p, size_t bytes, int) {
+    auto it = mem.find(uintptr_t(p));
+    CHECK(it != mem.end() && bytes <= it->second.bytes);  // inside the driver's block
+    if (it != mem.end()) it->second.cleared = true;
+    ++clears;
+    return kOk;
+  }
+  Error wait_clear(int) { return kOk; }
+  void forget_error() {}
+};
+using Cache = raptr::BlockCache<Model>;
+constexpr size_t MB = size_t(1) << 20;
+
+static void* get(Cache& c, size_t bytes) {
+  void* p = nullptr;
+  CHECK(c.malloc(&p, bytes) == Model::kOk);
+  auto it = c.driver().mem.find(uintptr_t(p));
+  CHECK(it != c.driver().mem.end() && it->second.bytes >= bytes &&
+        it->second.dev == c.driver().dev && it->second.cleared);
+  if (it != c.driver().mem.end()) it->second.cleared = false;  // the owner writes it
+  return p;
+}
+
+static void test_reuse() {
+  Cache c;
+  void* a = get(c, 9 * MB);
+  CHECK(c.free(a, false) == Model::kOk && c.driver().waits == 1 && c.driver().clears == 1);
+  CHECK(c.kept_bytes() == Cache::rounded(9 * MB));
+  CHECK(get(c, 9 * MB - 5) == a && c.kept_bytes() == 0);
+  CHECK(c.free(a, true) == Model::kOk && c.driver().waits == 1);
+  void* b = get(c, 5 * MB);  // less than four fifths of it: a block of its own
+  CHECK(b != a);
+  c.driver().dev = 1;  // the other device's
+  CHECK(get(c, 9 * MB) != a);
+  c.driver().dev = 0;
+  CHECK(get(c, 9 * MB) == a);
+  CHECK(c.free(nullptr, false) == Model::kOk);
+}
+
+static void test_freed_twice() {
+  Cache c;
+  void* a = get(c, 9 * MB);
+  CHECK(c.free(a, false) == Model::kOk);
+  CHECK(c.free(a, false) == Model::kInvalid);
+  void* b = get(c, 9 * MB);
+  CHECK(get(c, 9 * MB) != b);  // once only
+  CHECK(c.free(b, false) == Model::kOk && c.free(b, true) == Model::kInvalid);
+  int foreign = 0;
+  CHECK(c.free(&foreign, false) == Model::kInvalid);
+}
+
+// A block released with the driver's own call: whatever comes to its address
+// later is not the cache's.
+static void test_released_elsewhere() {
+  Cache c;
+  void* a = get(c, 9 * MB);
+  CHECK(c.driver().release(a) == Model::kOk);
+  c.driver().place(uintptr_t(a), 4096);
+  CHECK(c.free(a, false) == Model::kOk && c.driver().extent(a) == 0);  // the driver's free
+  CHECK(c.driver().clears == 0 && c.kept_bytes() == 0);
+  void* b = get(c, 9 * MB);
+  CHECK(c.free(b, false) == Model::kOk && c.driver().release(b) == Model::kOk);
+  CHECK(get(c, 9 * MB) != b && c.kept_bytes() == 0);  // a kept block that is gone
+  void* d = get(c, 9 * MB);
+  CHECK(c.free(d, false) == Model::kOk && c.driver().release(d) == Model::kOk);
+  c.driver().place(uintptr_t(d), 4096);
+  CHECK(c.free(d, false) == Model::kOk && c.driver().extent(d) == 0 && c.kept_bytes() == 0);
+}
+
+// The bound, the oldest first, and everything given back to find memory.
+static void test_bounds() {
+  Cache c;
+  std::vector<void*> p;
+  const size_t one = 512 * MB;
+  for (int k = 0; k < 12; ++k) p.push_back(get(c, one));
+  for (void* q : p) CHECK(c.free(q, false) == Model::kOk);
+  CHECK(c.kept_bytes() == Cache::kBytes && c.driver().releases == 4);
+  for (int k = 0; k < 4; ++k) CHECK(c.driver().extent(p[k]) == 0);
+  CHECK(c.driver().extent(p[4]) >= one);
+  c.driver().room = c.driver().used;  // no memory but the kept blocks'
+  void* big = get(c, 700 * MB);
+  CHECK(big && c.kept_bytes() == 0);
+  c.driver().room = c.driver().used;
+  void* none = &c;
+  CHECK(c.malloc(&none, 700 * MB) == Model::kNoMemory && !none);
+  CHECK(c.malloc(&none, Cache::kBlock + 1) == Model::kNoMemory && !none);
+  // larger blocks are the driver's alone
+  Cache d;
+  void* l = get(d, Cache::kBlock + 1);
+  CHECK(d.free(l, false) == Model::kOk && d.kept_bytes() == 0 && d.driver().used == 0);
+}
+
+// A device that cannot be waited for and one that is not current: the driver's
+// free, nothing kept.
+static void test_no_wait() {
+  Cache c;
+  void* a = get(c, 9 * MB);
+  c.driver().can_wait = false;
+  CHECK(c.free(a, false) == Model::kOk && c.kept_bytes() == 0 && c.driver().used == 0);
+  void* b = get(c, 9 * MB);
+  c.driver().can_wait = true;
+  c.driver().dev = 1;
+  CHECK(c.free(b, false) == Model::kOk && c.kept_bytes() == 0 && c.driver().used == 0);
+}
+
+int main() {
+  test_reuse();
+  test_freed_twice();
+  test_released_elsewhere();
+  test_bounds();
+  test_no_wait();
+  std::printf("%d failure(s)\n", failures);
+  return failures != 0;
+}
