@@ -46,9 +46,11 @@ inline hipStream_t S(raptr_stream_t s) { return reinterpret_cast<hipStream_t>(s)
 
 // ------------------------------------------------- device memory
 // hipMalloc and hipFree through a bounded cache of freed blocks (runtime.hip).
-// pool_free waits for the device, as hipFree does, unless the caller has.
+// pool_free waits for the device, as hipFree does, unless the caller has
+// (pool_wait: before several of them).
 hipError_t pool_malloc(void** p, size_t bytes);
 hipError_t pool_free(void* p, bool idle = false);
+hipError_t pool_wait();
 
 // ------------------------------------------------- workspace carving
 struct Carver {

@@ -4055,8 +4055,8 @@ int raptr_recon_destroy(raptr_recon* R) {
     return fail(RAPTR_ERR_INVALID_ARG, "plan has %d live clone(s): destroy them first",
                 R->nclones);
   clear_graphs(R);
-  if (!R->allocs.empty()) (void)hipDeviceSynchronize();
-  for (void* p : R->allocs) (void)pool_free(p, true);
+  const bool idle = !R->allocs.empty() && pool_wait() == hipSuccess;
+  for (void* p : R->allocs) (void)pool_free(p, idle);
   if (R->parent) --R->parent->nclones;
   delete R;
   return RAPTR_OK;

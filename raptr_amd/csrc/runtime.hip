@@ -68,7 +68,13 @@ struct HipDriver {
     (void)hipGetLastError();
     return 0;
   }
-  hipError_t wait() { return hipDeviceSynchronize(); }
+  // hipFree waits for the work of every stream, and leaves a capture that another
+  // thread has open as it is; hipDeviceSynchronize would invalidate it
+  hipError_t wait() {
+    void* p = nullptr;
+    const hipError_t e = hipMalloc(&p, 1);
+    return e == hipSuccess ? hipFree(p) : e;
+  }
   hipError_t clear(void* p, size_t bytes, int dev) {
     hipEvent_t& ev = cleared[dev];
     if (!ev) {
@@ -94,6 +100,11 @@ BlockCache<HipDriver>& cache() {
 
 hipError_t pool_malloc(void** p, size_t bytes) { return cache().malloc(p, bytes); }
 hipError_t pool_free(void* p, bool idle) { return cache().free(p, idle); }
+hipError_t pool_wait() {
+  const hipError_t e = cache().driver().wait();
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
+}
 
 }  // namespace raptr
 

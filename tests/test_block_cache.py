@@ -45,3 +45,65 @@ def test_handed_out_blocks_are_cleared(gpu):
             assert not a.numpy().any()
             a.copy_from(np.full(n, 0xA5, np.uint8))
             a.free()
+
+
+def _capture(stream, work, beside):
+    """work() captured on the stream in thread-local mode while beside() runs
+    in another thread; the capture's end status and the graph's nodes."""
+    import ctypes as C
+    import threading
+    H = C.CDLL("libamdhip64.so")
+    vp = C.c_void_p
+    failed = []
+
+    def run():
+        try:
+            beside()
+        except Exception as e:  # noqa: BLE001 - reported by the caller's assert
+            failed.append(e)
+    graph = vp()
+    assert H.hipStreamBeginCapture(vp(stream.handle), 1) == 0
+    work()
+    t = threading.Thread(target=run)
+    t.start()
+    t.join()
+    work()
+    status = H.hipStreamEndCapture(vp(stream.handle), C.byref(graph))
+    n = C.c_size_t()
+    if graph.value:
+        assert H.hipGraphGetNodes(graph, None, C.byref(n)) == 0
+        assert H.hipGraphDestroy(graph) == 0
+    assert not failed, failed
+    return status, n.value
+
+
+@pytest.mark.gpu
+def test_frees_leave_a_capture_of_another_thread(gpu):
+    """Blocks, and a plan with its blocks, freed while another thread captures:
+    the capture ends well and holds all of its work."""
+    import numpy as np
+    from raptr_amd import sysmat
+    from raptr_amd.device import DeviceArray, Stream
+    from raptr_amd.geometry import config_tiny
+    from raptr_amd.recon import Reconstructor
+    setup, grid, nrays = config_tiny()
+    A = sysmat.build_csr(setup, grid, np.arange(setup.nchannels, dtype=np.int32), nrays)
+    sens = sysmat.sensitivity(setup, grid, nrays)
+    R = Reconstructor(A, sens, "f32", 1, row_order=setup)
+    dy = DeviceArray.from_numpy(np.ones(A.m, np.float32))
+    dx = DeviceArray.from_numpy(np.full(A.n, 1.0 / A.n, np.float32))
+    st = Stream()
+
+    def work():
+        R.run(dy, dx, 1, use_graph=False, stream=st.handle)
+    blocks = [DeviceArray(n, np.uint8) for n in (1 << 12, 9 << 20, 64 << 20)]
+    plans = [Reconstructor(A, sens, "f32", 1, row_order=setup)]
+
+    def frees():
+        for b in blocks:
+            b.free()
+        plans.pop().close()
+        DeviceArray(9 << 20, np.uint8).free()  # a kept block, handed out and freed
+    status, alone = _capture(st, work, lambda: None)
+    assert status == 0 and alone >= 2
+    assert _capture(st, work, frees) == (0, alone)
