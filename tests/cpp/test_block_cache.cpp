@@ -149,10 +149,20 @@ static void test_bounds() {
   void* none = &c;
   CHECK(c.malloc(&none, 700 * MB) == Model::kNoMemory && !none);
   CHECK(c.malloc(&none, Cache::kBlock + 1) == Model::kNoMemory && !none);
-  // larger blocks are the driver's alone
+  // smaller and larger blocks are the driver's alone
   Cache d;
-  void* l = get(d, Cache::kBlock + 1);
-  CHECK(d.free(l, false) == Model::kOk && d.kept_bytes() == 0 && d.driver().used == 0);
+  for (size_t bytes : {size_t(1), Cache::kLeast - 1, Cache::kBlock + 1}) {
+    void* l = get(d, bytes);
+    CHECK(d.driver().used == bytes);
+    CHECK(d.free(l, false) == Model::kOk && d.kept_bytes() == 0 && d.driver().used == 0);
+    CHECK(d.free(l, false) == Model::kInvalid);
+  }
+  CHECK(d.driver().waits == 0 && d.driver().clears == 0);
+  for (size_t bytes : {Cache::kLeast, Cache::kLeast + 1, Cache::kBlock - 1, Cache::kBlock})
+    CHECK(d.free(get(d, bytes), false) == Model::kOk && d.kept_bytes() >= bytes);
+  c.driver().room = c.driver().used;  // a small one finds the kept blocks' memory too
+  CHECK(c.free(big, false) == Model::kOk && c.kept_bytes() > 0);
+  CHECK(get(c, 4096) && c.kept_bytes() == 0);
 }
 
 // A device that cannot be waited for and one that is not current: the driver's
