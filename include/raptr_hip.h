@@ -75,8 +75,14 @@ int raptr_version(void);
 int raptr_device_count(int* count);
 int raptr_set_device(int device);
 int raptr_device_name(char* buf, int len);
+/* raptr_free waits for the device and keeps blocks of 2 MiB to 1 GiB, cleared,
+ * for later allocations of the library (raptr_malloc and the plans'), up to
+ * 4 GiB per device.  They are given back when one of these finds no memory,
+ * and by raptr_release_cached, which a program calls before another allocator
+ * of the process needs them. */
 int raptr_malloc(void** ptr, size_t bytes);
 int raptr_free(void* ptr);
+int raptr_release_cached(void);
 int raptr_memcpy_h2d(void* dst, const void* src, size_t bytes, raptr_stream_t s);
 int raptr_memcpy_d2h(void* dst, const void* src, size_t bytes, raptr_stream_t s);
 int raptr_memcpy_d2d(void* dst, const void* src, size_t bytes, raptr_stream_t s);
@@ -96,6 +102,8 @@ int raptr_event_elapsed_ms(float* ms, void* start, void* stop);
 /* Work queued on s after this call waits for ev (hipStreamWaitEvent): joins
  * two streams' work, e.g. two plans run side by side. */
 int raptr_stream_wait_event(raptr_stream_t s, void* ev);
+/* free_bytes: the device's free memory and the blocks that raptr_free keeps
+ * (free to the library; to other allocators after raptr_release_cached). */
 int raptr_mem_info(size_t* free_bytes, size_t* total_bytes);
 
 /* ----------------------------------------------- geometry (host side) */

@@ -65,6 +65,7 @@ _SIGS = {
     "raptr_device_name": (i32, [C.c_char_p, i32]),
     "raptr_malloc": (i32, [P(vp), sz]),
     "raptr_free": (i32, [vp]),
+    "raptr_release_cached": (i32, []),
     "raptr_memcpy_h2d": (i32, [vp, vp, sz, vp]),
     "raptr_memcpy_d2h": (i32, [vp, vp, sz, vp]),
     "raptr_memcpy_d2d": (i32, [vp, vp, sz, vp]),

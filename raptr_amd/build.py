@@ -121,7 +121,7 @@ def build_cpp_tests():
     """C++ programs written against include/raptr/*.hpp, linked to the HIP
     library (rpath to raptr_amd/lib), and the host-only ones."""
     link = [f"-L{LIBDIR}", "-lraptr_hip", "-Wl,-rpath,$ORIGIN"]
-    for src, flags in [(s, link) for s in CPP_TESTS] + [(s, [f"-I{CSRC}"])
+    for src, flags in [(s, link) for s in CPP_TESTS] + [(s, [f"-I{CSRC}", "-pthread"])
                                                        for s in CPP_UNIT_TESTS]:
         out = os.path.join(LIBDIR, os.path.basename(src)[:-4])
         cmd = ["g++", "-O2", "-std=c++17", "-Wall", f"-I{os.path.join(ROOT, 'include')}", src,

@@ -6,7 +6,8 @@
 // of a 19 ms call in the driver, and 85 ms once the device's cleared memory is
 // used up, since the driver clears a freed block before it hands it out again.
 // Freed blocks of kLeast to kBlock bytes are kept, up to kBytes per device, the
-// oldest given back first, all of them when an allocation finds no memory.  A
+// oldest given back first, all of them when an allocation finds no memory or on
+// request (raptr_release_cached: other allocators cannot ask for them).  A
 // kept block is cleared when it is freed, so a caller sees what it saw before:
 // idle, cleared memory.  Sizes are rounded to eighths of a power of two, so that
 // lists of similar length find each other's blocks.
@@ -23,6 +24,7 @@
 #include <map>
 #include <mutex>
 #include <unordered_map>
+#include <utility>
 
 namespace raptr {
 
@@ -56,8 +58,8 @@ class BlockCache {
     Error e = d_.device(&dev);
     if (e != D::kOk) return e;
     const size_t need = ours ? rounded(bytes) : bytes;
-    std::lock_guard<std::mutex> lock(mu_);
     if (ours) {
+      std::lock_guard<std::mutex> lock(mu_);
       while (take(dev, need, p)) {
         Block& b = blocks_[*p];
         const bool there = d_.extent(*p) >= b.bytes;
@@ -65,33 +67,28 @@ class BlockCache {
         if (there && d_.wait_clear(dev) == D::kOk) return D::kOk;
         d_.forget_error();
         if (there) {
-          b.kept = true;
-          kept_.push_front(*p);
-          kept_bytes_[dev] += b.bytes;
+          keep(*p, b, true);
           *p = nullptr;
           break;
         }
         blocks_.erase(*p);  // released behind the cache's back
         *p = nullptr;
       }
-      e = d_.alloc(p, need);
-    } else {
-      e = D::kNoMemory;
     }
-    if (e == D::kNoMemory && kept_bytes_[dev]) {
+    size_t got = need;
+    e = ours ? d_.alloc(p, need) : D::kNoMemory;
+    if (e == D::kNoMemory && give_back(dev, 0)) {
       d_.forget_error();
-      for (auto it = kept_.begin(); it != kept_.end();)
-        if (blocks_[*it].dev == dev) {
-          (void)d_.release(*it);
-          blocks_.erase(*it);
-          it = kept_.erase(it);
-        } else {
-          ++it;
-        }
-      kept_bytes_[dev] = 0;
       e = d_.alloc(p, need);
     }
-    if (e == D::kOk && ours) blocks_[*p] = Block{need, dev, false};
+    if (e == D::kNoMemory && need > bytes) {  // without the rounding
+      d_.forget_error();
+      e = d_.alloc(p, got = bytes);
+    }
+    if (e == D::kOk && ours) {
+      std::lock_guard<std::mutex> lock(mu_);
+      blocks_[*p] = Block{got, dev, false};
+    }
     return e;
   }
 
@@ -127,25 +124,49 @@ class BlockCache {
       }
       return e;
     }
-    std::lock_guard<std::mutex> lock(mu_);
-    if (d_.clear(p, b.bytes, dev) != D::kOk) {
-      d_.forget_error();
-      return d_.release(p);
+    {
+      std::lock_guard<std::mutex> lock(mu_);
+      if (d_.clear(p, b.bytes, dev) != D::kOk) {
+        d_.forget_error();
+        return d_.release(p);
+      }
+      keep(p, b, false);
     }
-    b.kept = true;
-    blocks_[p] = b;
-    kept_.push_back(p);
-    kept_bytes_[dev] += b.bytes;
-    for (auto it = kept_.begin(); kept_bytes_[dev] > kBytes && it != kept_.end();)
-      if (blocks_[*it].dev == dev) {
-        kept_bytes_[dev] -= blocks_[*it].bytes;
-        (void)d_.release(*it);
+    (void)give_back(dev, kBytes);
+    return D::kOk;
+  }
+
+  // Kept blocks of a device given back to the driver, the oldest first, down to
+  // most bytes; the bytes given back.  (A release can wait for the device: the
+  // lock is not held meanwhile.)
+  size_t give_back(int dev, size_t most) {
+    std::list<std::pair<void*, Block>> out;
+    {
+      std::lock_guard<std::mutex> lock(mu_);
+      for (auto it = kept_.begin(); kept_bytes_[dev] > most && it != kept_.end();) {
+        const Block b = blocks_[*it];
+        if (b.dev != dev) {
+          ++it;
+          continue;
+        }
+        out.emplace_back(*it, b);
+        kept_bytes_[dev] -= b.bytes;
         blocks_.erase(*it);
         it = kept_.erase(it);
-      } else {
-        ++it;
       }
-    return D::kOk;
+    }
+    size_t bytes = 0;
+    for (auto& [p, b] : out) {
+      if (d_.release(p) == D::kOk) {
+        bytes += b.bytes;
+        continue;
+      }
+      d_.forget_error();
+      if (d_.extent(p) < b.bytes) continue;  // the driver's no more
+      std::lock_guard<std::mutex> lock(mu_);
+      keep(p, b, true);
+    }
+    return bytes;
   }
 
   // of the current device
@@ -164,6 +185,13 @@ class BlockCache {
     int dev;
     bool kept;  // freed by its owner, in kept_
   };
+
+  void keep(void* p, Block b, bool front) {
+    b.kept = true;
+    blocks_[p] = b;
+    kept_bytes_[b.dev] += b.bytes;
+    front ? kept_.push_front(p) : kept_.push_back(p);
+  }
 
   // the smallest kept block of the device with need bytes and at most a quarter
   // more, out of kept_

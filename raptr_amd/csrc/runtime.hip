@@ -255,7 +255,13 @@ int raptr_event_elapsed_ms(float* ms, void* a, void* b) {
 }
 int raptr_mem_info(size_t* free_bytes, size_t* total_bytes) {
   RAPTR_HIP_TRY(hipMemGetInfo(free_bytes, total_bytes));
-  if (free_bytes) *free_bytes += cache().kept_bytes();  // given back when needed
+  if (free_bytes) *free_bytes += cache().kept_bytes();
+  return RAPTR_OK;
+}
+int raptr_release_cached(void) {
+  int dev = 0;
+  RAPTR_HIP_TRY(hipGetDevice(&dev));
+  (void)cache().give_back(dev, 0);
   return RAPTR_OK;
 }
 

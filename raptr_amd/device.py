@@ -137,6 +137,11 @@ def synchronize():
     capi.call("raptr_device_sync")
 
 
+def release_cached():
+    """Blocks that freed arrays and plans left for reuse, back to the driver."""
+    capi.call("raptr_release_cached")
+
+
 def mem_info():
     f, t = C.c_size_t(), C.c_size_t()
     capi.call("raptr_mem_info", C.byref(f), C.byref(t))

@@ -4,7 +4,9 @@
 #include <cstdint>
 #include <cstdio>
 #include <map>
+#include <mutex>
 #include <set>
+#include <thread>
 #include <vector>
 
 #include "blockcache.hpp"
@@ -29,7 +31,7 @@ struct Model {
   uintptr_t next = 0x1000;
   size_t used = 0, room = size_t(64) << 30;
   int dev = 0, allocs = 0, releases = 0, waits = 0, clears = 0;
-  bool can_wait = true;
+  bool can_wait = true, can_release = true;
   Error device(int* d) {
     *d = dev;
     return kOk;
@@ -49,7 +51,7 @@ struct Model {
   }
   Error release(void* p) {
     auto it = mem.find(uintptr_t(p));
-    if (it == mem.end()) return kInvalid;
+    if (it == mem.end() || !can_release) return kInvalid;
     ++releases;
     used -= it->second.bytes;
     mem.erase(it);
@@ -146,6 +148,11 @@ static void test_bounds() {
   void* big = get(c, 700 * MB);
   CHECK(big && c.kept_bytes() == 0);
   c.driver().room = c.driver().used;
+  c.driver().room += 9 * MB - 17;  // room for the block but not for its rounding
+  void* tight = get(c, 9 * MB - 17);
+  CHECK(c.free(tight, false) == Model::kOk && c.kept_bytes() == 9 * MB - 17);
+  CHECK(c.give_back(0, 0) == 9 * MB - 17 && c.kept_bytes() == 0);
+  c.driver().room = c.driver().used;
   void* none = &c;
   CHECK(c.malloc(&none, 700 * MB) == Model::kNoMemory && !none);
   CHECK(c.malloc(&none, Cache::kBlock + 1) == Model::kNoMemory && !none);
@@ -178,12 +185,72 @@ static void test_no_wait() {
   CHECK(c.free(b, false) == Model::kOk && c.kept_bytes() == 0 && c.driver().used == 0);
 }
 
+// Everything given back on request, of one device; what the driver refuses to
+// release stays.
+static void test_give_back() {
+  Cache c;
+  void* a = get(c, 9 * MB);
+  void* b = get(c, 30 * MB);
+  c.driver().dev = 1;
+  void* other = get(c, 9 * MB);
+  CHECK(c.free(other, false) == Model::kOk);
+  c.driver().dev = 0;
+  CHECK(c.free(a, false) == Model::kOk && c.free(b, false) == Model::kOk);
+  c.driver().can_release = false;
+  CHECK(c.give_back(0, 0) == 0 && c.kept_bytes() >= 39 * MB);
+  c.driver().can_release = true;
+  CHECK(c.give_back(0, 0) >= 39 * MB && c.kept_bytes() == 0 && c.give_back(0, 0) == 0);
+  CHECK(c.free(a, false) == Model::kInvalid);
+  CHECK(c.driver().extent(other) && c.driver().mem.size() == 1);
+}
+
+// Four threads allocate, write and free blocks of a few sizes.
+static void test_threads() {
+  struct Locked : Model {
+    std::mutex mu;
+    Error alloc(void** p, size_t n) { std::lock_guard<std::mutex> l(mu); return Model::alloc(p, n); }
+    Error release(void* p) { std::lock_guard<std::mutex> l(mu); return Model::release(p); }
+    size_t extent(void* p) { std::lock_guard<std::mutex> l(mu); return Model::extent(p); }
+    Error wait() { std::lock_guard<std::mutex> l(mu); return Model::wait(); }
+    Error clear(void* p, size_t n, int d) { std::lock_guard<std::mutex> l(mu); return Model::clear(p, n, d); }
+  };
+  raptr::BlockCache<Locked> c;
+  c.driver().room = size_t(3) << 30;
+  std::mutex mu;
+  std::set<void*> out;
+  std::vector<std::thread> threads;
+  for (int t = 0; t < 4; ++t)
+    threads.emplace_back([&, t] {
+      for (int k = 0; k < 3000; ++k) {
+        void* p = nullptr;
+        const size_t n = (3 + (t * 7 + k * 13) % 11 * 40) * MB;
+        if (c.malloc(&p, n) != Model::kOk) continue;
+        {
+          std::lock_guard<std::mutex> l(mu);
+          CHECK(out.insert(p).second);  // nobody else's
+        }
+        std::this_thread::yield();
+        {
+          std::lock_guard<std::mutex> l(mu);
+          out.erase(p);
+        }
+        CHECK(c.free(p, k % 2) == Model::kOk);
+        if (k % 500 == 0) (void)c.give_back(0, 0);
+      }
+    });
+  for (auto& t : threads) t.join();
+  (void)c.give_back(0, 0);
+  CHECK(c.driver().used == 0 && c.kept_bytes() == 0);
+}
+
 int main() {
   test_reuse();
   test_freed_twice();
   test_released_elsewhere();
   test_bounds();
   test_no_wait();
+  test_give_back();
+  test_threads();
   std::printf("%d failure(s)\n", failures);
   return failures != 0;
 }

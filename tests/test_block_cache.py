@@ -107,3 +107,30 @@ def test_frees_leave_a_capture_of_another_thread(gpu):
     status, alone = _capture(st, work, lambda: None)
     assert status == 0 and alone >= 2
     assert _capture(st, work, frees) == (0, alone)
+
+
+@pytest.mark.gpu
+def test_cached_blocks_go_back_on_request(gpu):
+    """Free memory as the driver counts it: a freed block returns to it with
+    release_cached; mem_info counts it throughout."""
+    import ctypes as C
+    import numpy as np
+    from raptr_amd.device import DeviceArray, mem_info, release_cached
+    H = C.CDLL("libamdhip64.so")
+    f, t = C.c_size_t(), C.c_size_t()
+
+    def driver_free():
+        assert H.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+    # (the driver's count also moves by chunks of its own: blocks, half of one)
+    nb, half = 512 << 20, 256 << 20
+    release_cached()
+    before = driver_free()
+    a = DeviceArray(nb, np.uint8)
+    assert driver_free() <= before - half
+    held = mem_info()[0]
+    a.free()
+    assert driver_free() <= before - half
+    assert mem_info()[0] >= held + half
+    release_cached()
+    assert driver_free() >= before - half
