@@ -116,14 +116,18 @@ CPP_TESTS = [os.path.join(ROOT, "tests", "cpp", "test_reference_api.cpp")]
 # host-only programs over headers of csrc/, without the library
 CPP_UNIT_TESTS = [os.path.join(ROOT, "tests", "cpp", "test_block_cache.cpp")]
 
+# libraries that a test loads beside the library
+CPP_TEST_LIBS = [os.path.join(ROOT, "tests", "cpp", "failing_malloc.cpp")]
+
 
 def build_cpp_tests():
     """C++ programs written against include/raptr/*.hpp, linked to the HIP
     library (rpath to raptr_amd/lib), and the host-only ones."""
     link = [f"-L{LIBDIR}", "-lraptr_hip", "-Wl,-rpath,$ORIGIN"]
-    for src, flags in [(s, link) for s in CPP_TESTS] + [(s, [f"-I{CSRC}", "-pthread"])
-                                                       for s in CPP_UNIT_TESTS]:
-        out = os.path.join(LIBDIR, os.path.basename(src)[:-4])
+    for src, flags, ext in ([(s, link, "") for s in CPP_TESTS] +
+                            [(s, [f"-I{CSRC}", "-pthread"], "") for s in CPP_UNIT_TESTS] +
+                            [(s, ["-shared", "-fPIC", "-ldl"], ".so") for s in CPP_TEST_LIBS]):
+        out = os.path.join(LIBDIR, os.path.basename(src)[:-4]) + ext
         cmd = ["g++", "-O2", "-std=c++17", "-Wall", f"-I{os.path.join(ROOT, 'include')}", src,
                "-o", out + ".tmp"] + flags
         r = subprocess.run(cmd, capture_output=True, text=True)

@@ -3142,7 +3142,7 @@ int build_local_columns(raptr_recon* R, hipStream_t st, int rows_req = 0,
     int pick = nc - 1;
     int64_t* all = nullptr;
     if (at[nc] > 0) {
-      RAPTR_HIP_TRY(pool_malloc(reinterpret_cast<void**>(&all), size_t(at[nc]) * 8));
+      if ((rc = ralloc(R, &all, size_t(at[nc])))) return rc;
       for (int ci = 0; ci < nc; ++ci)
         if (at[ci + 1] > at[ci])
           hipLaunchKernelGGL(k_loc_union, dim3(unsigned(at[ci + 1] - at[ci])), dim3(256), shm, st,
@@ -3155,7 +3155,7 @@ int build_local_columns(raptr_recon* R, hipStream_t st, int rows_req = 0,
         le = hipMemcpyAsync(hc.data(), all, size_t(at[nc]) * 8, hipMemcpyDeviceToHost, st);
       if (le == hipSuccess) le = hipStreamSynchronize(st);
       if (le != hipSuccess) {
-        (void)pool_free(all);
+        rfree(R, all);
         return fail(RAPTR_ERR_DEVICE, "column unions: %s", hipGetErrorString(le));
       }
       double best = 1e30;
@@ -3177,7 +3177,7 @@ int build_local_columns(raptr_recon* R, hipStream_t st, int rows_req = 0,
     }
     rc = build_local_columns(R, st, kLocRowsChoices[pick],
                              at[pick + 1] > at[pick] ? all + at[pick] : nullptr);
-    (void)pool_free(all);
+    rfree(R, all);
     return rc;
   }
   const int rows = rows_req;
@@ -3210,7 +3210,7 @@ int build_local_columns(raptr_recon* R, hipStream_t st, int rows_req = 0,
     mx = hc.empty() ? 0 : *std::max_element(hc.begin(), hc.end());
     if (mx > kLocMaxUnion) {  // too spread out for LDS: the plan keeps no unions
       rfree(R, R->lup);
-      rfree(R, cnt);
+      if (!counted) rfree(R, cnt);
       return RAPTR_OK;
     }
   }
@@ -3223,7 +3223,7 @@ int build_local_columns(raptr_recon* R, hipStream_t st, int rows_req = 0,
   hipError_t le = hipGetLastError();
   if (le == hipSuccess) le = hipStreamSynchronize(st);
   if (le != hipSuccess) return fail(RAPTR_ERR_DEVICE, "column unions: %s", hipGetErrorString(le));
-  rfree(R, cnt);
+  if (!counted) rfree(R, cnt);
   R->lrows = rows;
   R->lmax = int(mx);
   R->lnu = h;
