@@ -886,8 +886,10 @@ __global__ __launch_bounds__(NW * kWave) void k_sm_rays(BuildArgs A) {
       }
     }
   }
-  if (lane == 0) s_cull[w] = 0;
-  if (cullw) s_cull[w] = 1;
+  // (one store a wave: the compiler keeps no order between the stores of
+  // different lanes to one word)
+  const int any_cull = __ballot(cullw) != 0u ? 1 : 0;
+  if (lane == 0) s_cull[w] = any_cull;
   __syncthreads();
 
   // Between the heads a ray is no farther from the channel's line than the

@@ -584,3 +584,23 @@ def test_mlem_f32_restatement(oracle):
     x64 = oracle.mlem_f64(rp, col, v32.astype(np.float64), yp, sens, x0, 5)
     assert float(np.sum(x32, dtype=np.float64)) == pytest.approx(1.0, abs=1e-5)
     assert np.linalg.norm(x32 - x64) / np.linalg.norm(x64) <= 1e-5
+
+
+@pytest.mark.parametrize("name,regu", [("along_y", False), ("same_heads", False), ("flat_z", True)])
+def test_ray_build_cases_need_the_cull(oracle, name, regu):
+    """The geometries that the ray-mask build is compared on hold rows whose
+    rays cross voxels outside the cylinder: a build that lost the test of
+    distance for one wave would keep them."""
+    from conftest import oracle_geom
+    from test_gpu_rays import CASES, _rows
+    setup, grid, nrays = CASES[name]
+    s, g = oracle_geom(oracle, setup, grid)
+    raygen = oracle.RAYGEN_REGU if regu else oracle.RAYGEN_RAND
+    v = np.arange(grid.nvox, dtype=np.int32)
+    outside = 0
+    for c in _rows(setup, 20):
+        val = oracle.sm_from_wq(s, g, np.full(grid.nvox, c, np.int32), v, nrays, raygen=raygen,
+                                seed=7)
+        val[oracle.workqueue(s, g, np.array([c], np.int32))[1]] = 0
+        outside += bool(val.any())
+    assert outside > 0
