@@ -623,7 +623,7 @@ int raptr_recon_get_broadcast(const raptr_recon* plan);
  * launch's row blocks into one shared image sum), kind 3 (the default) =
  * kind 2 with a backward in which each XCD takes one eighth of the row
  * blocks (a quarter, half or all of them on plans of few rows) and writes
- * its range's partial image (8 x n x 64 floats, allocated with the plan); a
+ * its range's partial image (n x 64 floats a range, allocated with the plan); a
  * fixed-order reduce adds them.  Shapes per G: 16: unroll
  * 8, 16 or 32, kind 2 or 3; 32: unroll 8 or 16, kind 3
  * (v_mfma_f32_32x32x2f32, 2 entries x 32 frames, whole 128-byte lines per
@@ -631,7 +631,10 @@ int raptr_recon_get_broadcast(const raptr_recon* plan);
  * Kinds 0 and 1 (vector FMAs with the keys and values in scalar
  * registers, groups of 4 and 8) were removed: the scalar-cache stream
  * capped them near 0.8 TB/s.  unroll applies to the forward (backward
- * steps are 8 entries).  get: group = G (0: no grouped layouts), fwd/
+ * steps are 8 entries): the entries a wave takes at a time from its group's
+ * list, or from its quarter of it with G = 16 and at most 8,192 groups, where a
+ * workgroup's four waves share a group (default 16 there and with G = 32, else
+ * 8).  get: group = G (0: no grouped layouts), fwd/
  * bwd_entries = union entries of each layout (lists padded to multiples of
  * 32 / 8). */
 int raptr_recon_set_grouped(raptr_recon* plan, int on, int unroll, int kind);

@@ -1173,7 +1173,7 @@ __global__ __launch_bounds__(256) void k_fwdm64(int64_t ng, int64_t m,
 // permutation), 2,484 of 2,200 301 -> 217; 8,826 of 465 191 and 189, 23,719 of
 // 1,280 1,106 and 1,137.
 constexpr int64_t kSplitGroups = 8192;
-template <int VT, int FB>
+template <int VT, int U, int FB>
 __global__ __launch_bounds__(256) void k_fwdm64s(int64_t ng, int64_t m,
                                                  const int64_t* __restrict__ gp,
                                                  const int* __restrict__ gcol,
@@ -1183,7 +1183,7 @@ __global__ __launch_bounds__(256) void k_fwdm64s(int64_t ng, int64_t m,
                                                  const float* __restrict__ y,
                                                  float* __restrict__ e) {
   using M = MF<16>;
-  constexpr int U = 4, E = M::K * U, NW = 256 / kWave;
+  constexpr int E = M::K * U, NW = 256 / kWave;
   __shared__ float part[NW][M::NR * FB][kWave];
   const int lane = threadIdx.x & (kWave - 1), w = wave_id();
   const int kq = lane / M::W, rw = lane % M::W;
@@ -2513,17 +2513,22 @@ int launch_fwd_any(const raptr_recon* R, int F, const float* x, const float* y, 
     const int GU = R->grp_unroll, GG = R->grp_g;
     const int FBA = R->fa / GG;
     if (GG == 16 && R->ngf <= kSplitGroups) {
-#define RAPTR_M64S(VV, FB_)                                                                  \
-      if (R->vt == VV && FBA == FB_)                                                         \
-        hipLaunchKernelGGL((k_fwdm64s<VV, FB_>), dim3(unsigned(R->ngf)), dim3(256), 0, st,    \
-                           R->ngf, m, R->gfp, R->gfcol,                                      \
-                           (const typename Val<VV>::T*)R->gfval, R->rscale, x, y, e);
-#define RAPTR_M64SV(VV) RAPTR_M64S(VV, 4) RAPTR_M64S(VV, 2) RAPTR_M64S(VV, 1)
+#define RAPTR_M64S(VV, UU, FB_)                                                              \
+      if (R->vt == VV && GU == MF<16>::K * UU && FBA == FB_) {                               \
+        hipLaunchKernelGGL((k_fwdm64s<VV, UU, FB_>), dim3(unsigned(R->ngf)), dim3(256), 0,    \
+                           st, R->ngf, m, R->gfp, R->gfcol,                                  \
+                           (const typename Val<VV>::T*)R->gfval, R->rscale, x, y, e);        \
+        RAPTR_LAUNCH_CHECK();                                                                \
+        return RAPTR_OK;                                                                     \
+      }
+#define RAPTR_M64SV(VV)                                                                      \
+  RAPTR_M64S(VV, 2, 4) RAPTR_M64S(VV, 4, 4) RAPTR_M64S(VV, 8, 4)                              \
+  RAPTR_M64S(VV, 2, 2) RAPTR_M64S(VV, 4, 2) RAPTR_M64S(VV, 8, 2)                              \
+  RAPTR_M64S(VV, 2, 1) RAPTR_M64S(VV, 4, 1) RAPTR_M64S(VV, 8, 1)
       RAPTR_M64SV(kF32) RAPTR_M64SV(kF16) RAPTR_M64SV(kBF16) RAPTR_M64SV(kU16)
 #undef RAPTR_M64SV
 #undef RAPTR_M64S
-      RAPTR_LAUNCH_CHECK();
-      return RAPTR_OK;
+      return fail(RAPTR_ERR_INVALID_ARG, "matrix-core forward shape unsupported");
     }
 #define RAPTR_M64(VV, G_, UU, FB_)                                                           \
     if (R->vt == VV && GG == G_ && GU == MF<G_>::K * UU && FBA == FB_) {                     \
@@ -3643,7 +3648,10 @@ int create_plan(raptr_recon** out, int m, int n, int64_t nnz, const int64_t* d_r
       }
       if (rc) return bail(rc);
       // default shape: matrix cores with per-XCD row ranges
-      R->grp_unroll = group == 16 ? 8 : 16;
+      // (k_fwdm64s with 8, 16 and 32 entries a step: 20,480 rows of 32^3 45, 45
+      // and 50 us, 39,730 of 52^3 219, 211 and 242, 20,000 of 96^3 705, 673 and
+      // 671, FP32)
+      R->grp_unroll = group == 16 && R->ngf > kSplitGroups ? 8 : 16;
       R->grp_pipe = 3;
       // kind 3's backward walks windows of about 131,072 rows per XCD and
       // launch (the best measured at full size for 16,384- and 32,768-row

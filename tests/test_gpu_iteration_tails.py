@@ -143,6 +143,45 @@ def test_frames64_both_forwards(gpu, rows, grid, vt):
     assert np.all(X[:, 63] == 0.0)
 
 
+@pytest.mark.parametrize("rows", [20011, 131089], ids=["split lists", "a wave a group"])
+@pytest.mark.parametrize("vt", ["f32", "f16", "bf16", "u16"])
+def test_frames64_every_forward_shape(gpu, rows, vt):
+    """Both forwards with each unroll, kind and number of active frames.  The
+    unroll is what the forward runs: with split lists it moves the cuts between
+    the waves, so some sums round otherwise."""
+    from raptr_amd import _capi as capi
+    from raptr_amd.device import DeviceArray
+    from raptr_amd.recon import Reconstructor
+    grid = centred_grid(7, 12.0)
+    A, dsens, _, _, y = _system(two_head_setup(13, 5, 36.0), grid, 4, rows=rows)
+    R = Reconstructor(A, dsens, vt, 64, row_order=two_head_setup(13, 5, 36.0), grid=grid)
+    split = (rows + 15) // 16 <= 8192
+    assert R.grouped()["unroll"] == (16 if split else 8)
+    Y = np.repeat(y[:, None], 64, axis=1)
+    Y[:, 1:] *= np.random.default_rng(4).integers(1, 4, (A.m, 63)).astype(np.float32)
+    X0 = np.repeat(_x0(grid.nvox)[:, None], 64, axis=1)
+    base = R.mlem(Y, X0, 3)
+    dy, ratios = DeviceArray.from_numpy(Y.reshape(-1)), {}
+    de = DeviceArray(A.m * 64, np.float32)
+    for unroll, kind in Reconstructor.GROUP_SHAPES[16]:
+        R.set_grouped(True, unroll, kind)
+        X = R.mlem(Y, X0, 3)
+        assert _rel(X, base) <= 1e-6, (unroll, kind)
+        for active in (16, 32) if kind == 3 else ():
+            dx = DeviceArray.from_numpy(X0.reshape(-1))
+            R.run(dy, dx, 3, 64, use_graph=False, active=active)
+            np.testing.assert_array_equal(dx.numpy().reshape(grid.nvox, 64)[:, :active],
+                                          X[:, :active], err_msg=f"{unroll} {kind} {active}")
+        dx = DeviceArray.from_numpy(base.reshape(-1))
+        capi.call("raptr_recon_forward", R.handle, 64, dx.ptr, dy.ptr, de.ptr, None)
+        ratios[unroll] = de.numpy()
+    for unroll in (16, 32):
+        assert _rel(ratios[unroll], ratios[8]) <= 1e-6
+    if split:
+        assert (ratios[32] != ratios[8]).any()
+    R.close()
+
+
 @pytest.mark.parametrize("n", [(64, 48, 49), (72, 66, 64), (96, 97, 64)])
 def test_frames64_few_ranges(gpu, n):
     """Grids of 9,408, 19,008 and 37,248 bricks under few rows: the backward
