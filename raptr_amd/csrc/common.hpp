@@ -284,7 +284,7 @@ __host__ __device__ inline float slab_length(const float* v, const float* r) {
 // reference lies in it.
 struct LineInterval {
   float p0[3], p1[3];
-  double u0, u1, u2, qa, rr;
+  double u0, u1, u2, qa, rr, inv_qa, inv_d;  // inv_qa: 1 / 2 qa
   __device__ LineInterval(const Geom& G, int cnl) {
     channel_centres(G, cnl, p0, p1);
     u0 = double(p1[0]) - double(p0[0]);
@@ -297,6 +297,8 @@ struct LineInterval {
     u2 *= il;
     rr = double(G.sumRadii) * (1.0 + 1e-4) + 1e-4;
     qa = u0 * u0 + u1 * u1;
+    inv_qa = 0.5 / qa;
+    inv_d = 1.0 / double(G.g.d[2]);
   }
   // number of voxels of the column that may pass, the first at lo
   __device__ int column(const raptr_grid_t& g, int ix, int iy, int& lo) const {
@@ -314,10 +316,10 @@ struct LineInterval {
       const double disc = qb * qb - 4.0 * qa * qc;
       if (disc >= 0.0) {
         const double sq = sqrt(disc);
-        const double z1 = double(p0[2]) + (-qb - sq) / (2.0 * qa);
-        const double z2 = double(p0[2]) + (-qb + sq) / (2.0 * qa);
-        const double f1 = (z1 - double(g.o[2])) / double(g.d[2]) - 0.5;
-        const double f2 = (z2 - double(g.o[2])) / double(g.d[2]) - 0.5;
+        const double z1 = double(p0[2]) + (-qb - sq) * inv_qa;
+        const double z2 = double(p0[2]) + (-qb + sq) * inv_qa;
+        const double f1 = (z1 - double(g.o[2])) * inv_d - 0.5;
+        const double f2 = (z2 - double(g.o[2])) * inv_d - 0.5;
         lo = int(fmax(floor(f1) - 1.0, 0.0));
         hi = int(fmin(ceil(f2) + 1.0, double(nz - 1)));
       }
