@@ -279,9 +279,12 @@ __host__ __device__ inline float slab_length(const float* v, const float* r) {
 
 // The cull by voxel columns.  The centres of column (ix, iy) closer to a
 // channel's line than the radius form one z interval (a convex set meets a
-// line in an interval); it is found in FP64, widened by a relative radius slack
-// and one voxel at each end, so every voxel that passes the float test of the
-// reference lies in it.
+// line in an interval); it is found in FP64 and widened by one voxel at each end
+// and by a slack of the radius, so every voxel that passes the float test of the
+// reference lies in it.  That test's rounding grows with the coordinates: the
+// centre, the differences to a pixel centre, the products of the cross product
+// over the line's length, each below 2^-24 of a few times the largest of them,
+// 4e-6 of it in all (u: qa < 1e-12 adds 2e-6); the slack is 8e-6.
 struct LineInterval {
   float p0[3], p1[3];
   double u0, u1, u2, qa, rr, inv_qa, inv_d;  // inv_qa: 1 / 2 qa
@@ -295,7 +298,13 @@ struct LineInterval {
     u0 *= il;
     u1 *= il;
     u2 *= il;
-    rr = double(G.sumRadii) * (1.0 + 1e-4) + 1e-4;
+    double far = 0.0;
+    for (int k = 0; k < 3; ++k) {
+      far = fmax(far, fmax(fabs(double(p0[k])), fabs(double(p1[k]))));
+      const double o = double(G.g.o[k]);
+      far = fmax(far, fmax(fabs(o), fabs(o + double(G.g.n[k]) * double(G.g.d[k]))));
+    }
+    rr = double(G.sumRadii) * (1.0 + 1e-4) + 1e-4 + 8e-6 * far;
     qa = u0 * u0 + u1 * u1;
     inv_qa = 0.5 / qa;
     inv_d = 1.0 / double(G.g.d[2]);

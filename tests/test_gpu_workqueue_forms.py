@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from conftest import oracle_geom
+from raptr_amd.geometry import MeasurementSetup, VoxelGrid
 from test_gpu_rays import CASES
 
 pytestmark = pytest.mark.gpu
@@ -79,3 +80,25 @@ def test_pair_values_any_order(gpu, oracle, raygen, length, order):
     want[bad | (vox == grid.nvox)] = 0
     np.testing.assert_array_equal(sysmat.sm_from_wq(setup, grid, cnl, vox, nrays, seed=3,
                                                     raygen=rg), want)
+
+
+@pytest.mark.parametrize("v,o1", [(2.504554271697998, 99406.609375),
+                                  (2.5129311084747314, 99405.75),
+                                  (2.521639347076416, 99403.3359375)])
+def test_coordinates_that_round_coarsely(gpu, oracle, v, o1):
+    """Heads 900 mm apart with 20,000 rows of 10 um pixels, in um: the centres
+    round by more than a ten-thousandth of the cull's radius, and a voxel
+    outside it by FP64 passes the float test."""
+    from raptr_amd import sysmat
+    ny = 20000
+    setup = MeasurementSetup(-450e3, 450e3, 1, 1, ny, 1, ny, 0.0, 10.0, 10.0, 10.0)
+    grid = VoxelGrid((-0.5 * v, o1, -1.5 * v), (v, v, v), (1, 200, 4))
+    s, g = oracle_geom(oracle, setup, grid)
+    c = setup.lin_id(0, ny - 35, 0, ny - 35, 0)
+    want = oracle.workqueue(s, g, np.array([c], np.int32))[1]
+    lst = np.full(4100, c, np.int32)
+    got = sysmat.workqueue(setup, grid, lst)
+    np.testing.assert_array_equal(got[1], np.tile(want, len(lst)))
+    np.testing.assert_array_equal(sysmat.workqueue_counts(setup, grid, lst), len(want))
+    A = sysmat.build_csr(setup, grid, lst[:3], 4, keep_zeros=True).to_host()
+    np.testing.assert_array_equal(A[1], np.tile(want, 3))
