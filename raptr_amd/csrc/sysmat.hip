@@ -127,18 +127,33 @@ __global__ __launch_bounds__(256) void k_sm_from_wq(Geom G, const int* cnl, cons
 // k_sm_from_wq for queues in channel order (as raptr_workqueue writes them):
 // a workgroup's kWqChunk pairs hold few channels, so it makes a channel's rays
 // and plane tables (as k_sm_build's) once in LDS for all of its pairs; a chunk of
-// more than kWqRuns runs takes k_sm_from_wq's way, rays anew for every pair.
+// more than max_runs runs takes k_sm_from_wq's way, rays anew for every pair.
 // The terms are slab_length's: a ray that misses the voxel adds +0.  8.4M
 // pairs of 3,000 channels, 10 rays, 32^3 voxels: 519 -> 97 us,
 // bound by the VALU of the ten slab tests.
 constexpr int kWqChunk = 1024;
-constexpr int kWqRuns = 6;
+
+// Runs of a chunk up to which the shared tables pay; 0: not for this call.
+// Measured with 2M pairs (us, p planes): pairs alone 15 + 10.5 nrays; shared 8 +
+// 1.2 nrays and 8 + 0.0018 nrays p for each run, so 2, 10 and 21 runs with 1, 10
+// and 30 rays of 99 planes (12 runs of 10 rays 134 shared, 122 alone; 16 of 30
+// 262 and 321), 2, 7 and 12 with 291 (8 runs of 10 rays 120 and 119, 12 of 30 336
+// and 318).  On short queues the tables' serial steps outlast the pairs: 65,536
+// pairs, 10 rays, 32^3 voxels 9 us alone and 15 shared, 262,144 of 96^3 19 and 19
+// to 26, 1M of 256^3 61 and 37 to 49; but many rays of one pair are as serial (64
+// pairs, 30 rays, 32^3: 19 and 10).
+inline int wq_max_runs(int64_t n, int nrays, int planes) {
+  const bool few = n <= 256 && nrays >= 16;
+  if (!few && double(n) * nrays < 4e6 + 8e3 * planes) return 0;
+  return int((7.5 + 9.3 * nrays) / (8.0 + 0.0018 * double(nrays) * planes));
+}
 
 __global__ __launch_bounds__(256) void k_sm_from_wq_runs(Geom G, const int* __restrict__ cnl,
                                                          const int* __restrict__ vxl,
                                                          float* __restrict__ val, int64_t n,
                                                          int nrays, uint32_t seed, int raygen,
-                                                         int stride, FastDiv div_yz,
+                                                         int max_runs, int stride,
+                                                         FastDiv div_yz,
                                                          FastDiv div_z) {
   constexpr int PER = kWqChunk / 256;
   extern __shared__ float wq_lds[];
@@ -172,7 +187,7 @@ __global__ __launch_bounds__(256) void k_sm_from_wq_runs(Geom G, const int* __re
   if (lane == 0) s_runs[w] = runs;
   if (t == 0) s_next = kWqChunk;
   __syncthreads();
-  if (s_runs[0] + s_runs[1] + s_runs[2] + s_runs[3] > kWqRuns) {
+  if (s_runs[0] + s_runs[1] + s_runs[2] + s_runs[3] > max_runs) {
 #pragma unroll 1
     for (int k = 0; k < PER; ++k) {
       const int64_t i = base + k * 256 + t;
@@ -1300,10 +1315,12 @@ int raptr_sm_from_wq(const raptr_setup_t* setup, const raptr_grid_t* grid, const
   const int pl = grid->n[0] + grid->n[1] + grid->n[2] + 3, stride = (pl + 1) | 1;
   const size_t lds = size_t(nrays) * (8 + size_t(stride)) * sizeof(float);
   const int64_t chunks = (wq_length + kWqChunk - 1) / kWqChunk;
+  const int max_runs = wq_max_runs(wq_length, nrays, pl);
   // rays per channel whose tables leave a CU two workgroups or more
-  if (raygen != RAPTR_RAYGEN_RAND_ELEMENT && lds <= 64 * 1024 && chunks < (1 << 22)) {
+  if (raygen != RAPTR_RAYGEN_RAND_ELEMENT && lds <= 64 * 1024 && chunks < (1 << 22) &&
+      max_runs > 0) {
     hipLaunchKernelGGL(k_sm_from_wq_runs, dim3(unsigned(chunks)), dim3(256), lds, S(stream), G,
-                       d_cnl, d_vxl, d_val, wq_length, nrays, seed, raygen, stride,
+                       d_cnl, d_vxl, d_val, wq_length, nrays, seed, raygen, max_runs, stride,
                        make_fastdiv(uint32_t(grid->n[1] * grid->n[2])),
                        make_fastdiv(uint32_t(grid->n[2])));
     RAPTR_LAUNCH_CHECK();

@@ -82,6 +82,37 @@ def test_pair_values_any_order(gpu, oracle, raygen, length, order):
                                                     raygen=rg), want)
 
 
+@pytest.mark.parametrize("name,length", [("ragged", 560001), ("rays_32", 1), ("rays_32", 255),
+                                         ("rays_32", 256), ("rays_32", 150001)])
+@pytest.mark.parametrize("order", ["runs", "few", "most", "one more", "shuffled"])
+def test_pair_values_by_runs(gpu, oracle, name, length, order):
+    """Queues whose chunks share a channel's rays: long ones, and short ones of
+    many rays; chunks of one run, of as many as share (9 with 9 rays and 74
+    planes, 27 with 32 and 51) and of one more."""
+    from raptr_amd import sysmat
+    setup, grid, nrays = CASES[name]
+    s, g = oracle_geom(oracle, setup, grid)
+    most = int((7.5 + 9.3 * nrays) / (8 + 0.0018 * nrays * (sum(grid.n) + 3)))
+    assert most == {"ragged": 9, "rays_32": 27}[name]
+    rng = np.random.default_rng(length)
+    vox = rng.integers(0, grid.nvox, length).astype(np.int32)
+    pool = rng.choice(setup.nchannels, 64, replace=False).astype(np.int32)
+    pos = np.arange(length)
+    chunk = min(1024, length)
+
+    def runs(k):
+        return pool[(pos // chunk + pos % chunk * k // chunk) % 64]
+    cnl = {"runs": pool[pos // 1500 % 64], "few": runs(3), "most": runs(most),
+           "one more": runs(most + 1),
+           "shuffled": rng.permutation(np.resize(pool, length))}[order].astype(np.int32)
+    want = oracle.sm_from_wq(s, g, cnl, vox, nrays, seed=3)
+    np.testing.assert_array_equal(sysmat.sm_from_wq(setup, grid, cnl, vox, nrays, seed=3), want)
+    bad = rng.random(length) < 0.001
+    cnl[bad] = rng.choice([-1, setup.nchannels, 2**31 - 1], int(bad.sum()))
+    want[bad] = 0
+    np.testing.assert_array_equal(sysmat.sm_from_wq(setup, grid, cnl, vox, nrays, seed=3), want)
+
+
 @pytest.mark.parametrize("v,o1", [(2.504554271697998, 99406.609375),
                                   (2.5129311084747314, 99405.75),
                                   (2.521639347076416, 99403.3359375)])
