@@ -7,20 +7,25 @@ namespace raptr {
 namespace {
 
 constexpr int kRsBlock = 256;
-constexpr int kRsItems = 16;  // per thread
-constexpr int kRsTile = kRsBlock * kRsItems;
+// Pairs of a thread: 16, and 8 in short sorts, where the serial steps of a tile
+// are what a pass waits for.  coo_sort of 5,000 pairs 119 us with 16 and 104 with
+// 8, 100,000 200 and 187, 1M 700 and 691, 2M 753 and 754, 8M 997 and 1,029, 30M
+// 2,131 and 2,316.
+constexpr int kRsItems = 16, kRsFewItems = 8;
+constexpr int kRsTile = kRsBlock * kRsFewItems;  // scratch is laid out for these
+constexpr int64_t kRsShort = int64_t(1) << 20;
 constexpr int kRsBins = 256;
 constexpr int kRsWaves = kRsBlock / kWave;
 
-template <class K>
+template <class K, int ITEMS>
 __global__ __launch_bounds__(kRsBlock) void k_rs_hist(const K* keys, int64_t n, int shift,
                                                       uint32_t* hist, int ntiles) {
   __shared__ uint32_t h[kRsBins];
   h[threadIdx.x] = 0;
   __syncthreads();
-  int64_t base = int64_t(blockIdx.x) * kRsTile;
+  int64_t base = int64_t(blockIdx.x) * (kRsBlock * ITEMS);
 #pragma unroll
-  for (int r = 0; r < kRsItems; ++r) {
+  for (int r = 0; r < ITEMS; ++r) {
     int64_t p = base + r * kRsBlock + threadIdx.x;
     if (p < n) atomicAdd(&h[uint32_t(keys[p] >> shift) & 0xff], 1u);
   }
@@ -28,7 +33,7 @@ __global__ __launch_bounds__(kRsBlock) void k_rs_hist(const K* keys, int64_t n, 
   hist[int64_t(threadIdx.x) * ntiles + blockIdx.x] = h[threadIdx.x];
 }
 
-// Stable scatter of one tile.  A wave takes 1,024 consecutive pairs, 64 at a
+// Stable scatter of one tile.  A wave takes a quarter of its pairs in a row, 64 at a
 // time: a pair's rank is the wave's running count of its digit plus its rank
 // among the equal-digit lanes (found with 8 ballots), with no barrier between
 // the rounds.  Then the digits' counts are added over waves and digits, the
@@ -36,24 +41,24 @@ __global__ __launch_bounds__(kRsBlock) void k_rs_hist(const K* keys, int64_t n, 
 // that a digit's run goes out in whole lines.  (Rounds of 256 pairs, four
 // barriers each, written straight from the lanes: 31M 12-byte pairs 0.40 ms a
 // pass, now 0.18.)
-template <class K, class V>
+template <class K, class V, int ITEMS>
 __global__ __launch_bounds__(kRsBlock) void k_rs_scatter(const K* kin, const V* vin, int64_t n,
                                                          int shift, const uint32_t* offs,
                                                          int ntiles, K* kout, V* vout) {
   __shared__ uint32_t wc[kRsWaves][kRsBins];
   __shared__ uint32_t s_tile[kRsBins], s_run[kRsBins];
   __shared__ int s_scan[kRsWaves];
-  __shared__ uint8_t s_dig[kRsTile];
-  __shared__ uint64_t s_buf[kRsTile];
+  __shared__ uint8_t s_dig[kRsBlock * ITEMS];
+  __shared__ uint64_t s_buf[kRsBlock * ITEMS];
   const int t = threadIdx.x, w = t / kWave, lane = t & (kWave - 1);
-  const int64_t base = int64_t(blockIdx.x) * kRsTile;
-  const int64_t first = base + w * (kRsItems * kWave) + lane;
+  const int64_t base = int64_t(blockIdx.x) * (kRsBlock * ITEMS);
+  const int64_t first = base + w * (ITEMS * kWave) + lane;
   const uint32_t off = offs[int64_t(t) * ntiles + blockIdx.x];
-  K key[kRsItems];
-  V val[kRsItems];
-  uint32_t rank[kRsItems];
+  K key[ITEMS];
+  V val[ITEMS];
+  uint32_t rank[ITEMS];
 #pragma unroll
-  for (int r = 0; r < kRsItems; ++r) {
+  for (int r = 0; r < ITEMS; ++r) {
     const int64_t p = first + r * kWave;
     key[r] = p < n ? kin[p] : K(0);
     val[r] = p < n ? vin[p] : V(0);
@@ -62,7 +67,7 @@ __global__ __launch_bounds__(kRsBlock) void k_rs_scatter(const K* kin, const V* 
   for (int ww = 0; ww < kRsWaves; ++ww) wc[ww][t] = 0;
   __syncthreads();
 #pragma unroll
-  for (int r = 0; r < kRsItems; ++r) {
+  for (int r = 0; r < ITEMS; ++r) {
     const bool valid = first + r * kWave < n;
     const uint32_t digit = uint32_t(key[r] >> shift) & 0xff;
     uint64_t m = __ballot(valid);
@@ -95,7 +100,7 @@ __global__ __launch_bounds__(kRsBlock) void k_rs_scatter(const K* kin, const V* 
   __syncthreads();
   K* bk = reinterpret_cast<K*>(s_buf);
 #pragma unroll
-  for (int r = 0; r < kRsItems; ++r) {
+  for (int r = 0; r < ITEMS; ++r) {
     const uint32_t digit = uint32_t(key[r] >> shift) & 0xff;
     rank[r] += s_tile[digit] + wc[w][digit];
     if (first + r * kWave < n) {
@@ -108,7 +113,7 @@ __global__ __launch_bounds__(kRsBlock) void k_rs_scatter(const K* kin, const V* 
   __syncthreads();
   V* bv = reinterpret_cast<V*>(s_buf);
 #pragma unroll
-  for (int r = 0; r < kRsItems; ++r)
+  for (int r = 0; r < ITEMS; ++r)
     if (first + r * kWave < n) bv[rank[r]] = val[r];
   __syncthreads();
   for (int i = t; i < tot; i += kRsBlock) vout[s_run[s_dig[i]] + uint32_t(i)] = bv[i];
@@ -148,6 +153,21 @@ bool take_sort(Carver& c, int64_t n, SortBufs* b) {
   return c.ok;
 }
 
+// One pass: (kin, vin) to (kout, vout) by the digit at shift.
+template <class K, class V, int ITEMS>
+int radix_pass(const K* kin, const V* vin, K* kout, V* vout, uint32_t* hist, uint32_t* offs,
+               void* scan_ws, size_t scan_bytes, int64_t n, int shift, hipStream_t st) {
+  const int64_t ntiles = (n + kRsBlock * ITEMS - 1) / (kRsBlock * ITEMS);
+  hipLaunchKernelGGL((k_rs_hist<K, ITEMS>), dim3(unsigned(ntiles)), dim3(kRsBlock), 0, st, kin, n,
+                     shift, hist, int(ntiles));
+  RAPTR_LAUNCH_CHECK();
+  RAPTR_TRY(scan_exclusive_u32(hist, offs, ntiles * kRsBins, nullptr, scan_ws, scan_bytes, st));
+  hipLaunchKernelGGL((k_rs_scatter<K, V, ITEMS>), dim3(unsigned(ntiles)), dim3(kRsBlock), 0, st,
+                     kin, vin, n, shift, (const uint32_t*)offs, int(ntiles), kout, vout);
+  RAPTR_LAUNCH_CHECK();
+  return RAPTR_OK;
+}
+
 // Sorts (k[0], v[0]) by bits [0, bits) of the key; *result: the buffer index
 // holding the sorted pairs.
 template <class K, class V>
@@ -156,16 +176,10 @@ int radix_sort_kv(K* const (&k)[2], V* const (&v)[2], uint32_t* hist, uint32_t* 
                   int* result) {
   int cur = 0;
   if (n > int64_t(UINT32_MAX)) return fail(RAPTR_ERR_INVALID_ARG, "sort length exceeds 2^32");
-  int64_t ntiles = (n + kRsTile - 1) / kRsTile;
+  const auto pass = n <= kRsShort ? radix_pass<K, V, kRsFewItems> : radix_pass<K, V, kRsItems>;
   for (int shift = 0; shift < bits; shift += 8) {
-    hipLaunchKernelGGL(k_rs_hist<K>, dim3(unsigned(ntiles)), dim3(kRsBlock), 0, st,
-                       (const K*)k[cur], n, shift, hist, int(ntiles));
-    RAPTR_LAUNCH_CHECK();
-    RAPTR_TRY(scan_exclusive_u32(hist, offs, ntiles * kRsBins, nullptr, scan_ws, scan_bytes, st));
-    hipLaunchKernelGGL((k_rs_scatter<K, V>), dim3(unsigned(ntiles)), dim3(kRsBlock), 0, st,
-                       (const K*)k[cur], (const V*)v[cur], n, shift, (const uint32_t*)offs,
-                       int(ntiles), k[cur ^ 1], v[cur ^ 1]);
-    RAPTR_LAUNCH_CHECK();
+    RAPTR_TRY(pass(k[cur], v[cur], k[cur ^ 1], v[cur ^ 1], hist, offs, scan_ws, scan_bytes, n,
+                   shift, st));
     cur ^= 1;
   }
   *result = cur;
