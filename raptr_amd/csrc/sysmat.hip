@@ -23,6 +23,7 @@
 //         dropped with a second ballot compaction into an LDS row buffer;
 //      4. row buffers are flushed as pieces into a staging area and packed
 //         into a CSR with 64-bit row pointers per channel chunk.
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <mutex>
@@ -289,8 +290,9 @@ struct Piece {
 // One staging counter for all rows serialises the workgroups (two additions
 // to one cache line took 25 ns a row, as long as the row itself), so large
 // launches spread their rows over kAreas counters in separate lines.
-constexpr int kAreas = 64;
+constexpr int kAreas = kWave;  // (k_rowptr_fill: a lane each)
 constexpr int kCountStride = 16;  // counters are 128 bytes apart
+static_assert(sizeof(Piece) == 24, "the piece table's entries");
 
 struct BuildArgs {
   Geom G;
@@ -1144,10 +1146,20 @@ __global__ void k_clear_counts(unsigned long long* a, int na, unsigned long long
   for (int i = threadIdx.x; i < nb; i += blockDim.x) b[i] = 0;
 }
 
-// row_ptr[i] = base + excl[i], i < rows; row_ptr[rows] = base + *sum
+// row_ptr[i] = base + excl[i], i < rows; row_ptr[rows] = base + *sum; and (st_count
+// given) the entries that the fullest of the staging areas was asked for
 __global__ void k_rowptr_fill(const int64_t* excl, const int64_t* sum, int rows, int64_t base,
-                              int64_t* row_ptr) {
+                              int64_t* row_ptr, const unsigned long long* st_count,
+                              unsigned long long* most) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (st_count && i < kAreas) {  // the first wave
+    unsigned long long v = st_count[i * kCountStride];
+    for (int j = kWave / 2; j > 0; j >>= 1) {
+      const unsigned long long o = __shfl_xor(v, j, kWave);
+      v = o > v ? o : v;
+    }
+    if (i == 0) *most = v;
+  }
   if (i < rows) row_ptr[i] = base + excl[i];
   if (i == 0) row_ptr[rows] = base + *sum;
 }
@@ -1409,13 +1421,15 @@ int raptr_sm_build_csr_ex(const raptr_setup_t* setup, const raptr_grid_t* grid,
   A.piece_count = reinterpret_cast<unsigned*>(&counters[0]);
   A.flags = reinterpret_cast<unsigned*>(&counters[1]);
   A.pieces = pieces;
-  A.piece_cap = int(L.piece_cap);
+  // the staging areas' counters: the end of the piece table, from a line on
+  const size_t area_at =
+      (size_t(L.piece_cap) * 24 - kAreas * kCountStride * sizeof(unsigned long long)) & ~size_t(127);
+  unsigned long long* area_counts =
+      reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(pieces) + area_at);
+  A.piece_cap = int(area_at / sizeof(Piece));
 
   int64_t total = 0;
   int first = 0;
-  // of the staging that a chunk's entries should fill (k_sm_rays asks for a
-  // fourth to a half more than they)
-  double share = 0.6;
   // the first chunk measures the density: rows of up to 4,096 entries fit
   int64_t rows0 = staging >> 12;
   if (rows0 < 64) rows0 = 64;
@@ -1426,10 +1440,9 @@ int raptr_sm_build_csr_ex(const raptr_setup_t* setup, const raptr_grid_t* grid,
     A.first = first;
     A.rows = rows;
     // few rows may fill the staging unevenly: one area
-    // (kAreas counters lie in the row offsets, which are made afterwards)
     A.areas = rows >= kAreas * kCountStride ? kAreas : 1;
     A.st_cap = staging / A.areas;
-    A.st_count = A.areas > 1 ? reinterpret_cast<unsigned long long*>(excl) : &counters[3];
+    A.st_count = A.areas > 1 ? area_counts : &counters[3];
     hipLaunchKernelGGL(k_clear_counts, dim3(1), dim3(256), 0, st, counters, 4, A.st_count,
                        A.areas > 1 ? kAreas * kCountStride : 0);
     RAPTR_LAUNCH_CHECK();
@@ -1441,9 +1454,10 @@ int raptr_sm_build_csr_ex(const raptr_setup_t* setup, const raptr_grid_t* grid,
                                      scan_ws, sb, st));
     hipLaunchKernelGGL(k_rowptr_fill, dim3(grid_for(rows, 256)), dim3(256), 0, st,
                        (const int64_t*)excl, (const int64_t*)&counters[2], rows, total,
-                       d_row_ptr + first);
+                       d_row_ptr + first,
+                       A.areas > 1 ? (const unsigned long long*)area_counts : nullptr, &counters[3]);
     RAPTR_LAUNCH_CHECK();
-    unsigned long long hc[3];
+    unsigned long long hc[4];
     RAPTR_HIP_TRY(hipMemcpyAsync(hc, counters, sizeof(hc), hipMemcpyDeviceToHost, st));
     RAPTR_HIP_TRY(hipStreamSynchronize(st));
     if (unsigned(hc[1] & 0xffffffffu)) {
@@ -1454,8 +1468,9 @@ int raptr_sm_build_csr_ex(const raptr_setup_t* setup, const raptr_grid_t* grid,
         A.by_candidate = 1;
         continue;
       }
-      rows = rows / 2;
-      share *= 0.5;
+      // the rows that would have fitted at what these asked for (of pieces: half)
+      const double fit = hc[3] > uint64_t(A.st_cap) ? 0.9 * double(A.st_cap) / double(hc[3]) : 0.5;
+      rows = std::max(1, std::min(rows - 1, int(rows * fit)));
       continue;
     }
     A.by_candidate = 0;
@@ -1472,9 +1487,10 @@ int raptr_sm_build_csr_ex(const raptr_setup_t* setup, const raptr_grid_t* grid,
     }
     total += chunk_nnz;
     first += rows;
-    // next chunk: fill that share of the staging at the observed density
-    double avg = rows ? double(chunk_nnz) / rows : 0.0;
-    int64_t want = avg > 0 ? int64_t(share * double(staging) / avg) : max_rows;
+    // next chunk: four fifths of the staging at what these rows asked for (a
+    // count: 0.6 of it at their entries)
+    const double asked = fill ? double(hc[3]) * A.areas : double(chunk_nnz) * (0.8 / 0.6);
+    int64_t want = asked > 0 ? int64_t(0.8 * double(staging) * rows / asked) : max_rows;
     if (want > max_rows) want = max_rows;
     if (want < 1) want = 1;
     rows = int(want);

@@ -126,3 +126,22 @@ def test_build_kernels_meet(gpu, oracle):
     got = sysmat.build_csr(setup, grid, lst, 4).to_host()
     for a, b in zip(got, (rp, col, val)):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("staging", [1 << 14, 1 << 17, 1 << 19])
+def test_staging_areas(gpu, oracle, staging):
+    """Lists whose chunks reach the 64 staging areas (1,024 rows) and overflow
+    them: rows outside the grid, then long rows, then rows of both kinds."""
+    from raptr_amd import sysmat
+    setup, grid = two_head_setup(6, 5, 36.0), centred_grid(24, 0.5)
+    s, g = oracle_geom(oracle, setup, grid)
+    every = np.arange(setup.nchannels, dtype=np.int32)
+    n = np.diff(oracle.build_csr(s, g, every, 6, seed=3)[0])
+    order = np.argsort(n, kind="stable").astype(np.int32)
+    rng = np.random.default_rng(2)
+    lst = np.concatenate([order[:3000], order[-1500:], rng.permutation(order)]).astype(np.int32)
+    assert n[order[:1500]].max() == 0 and n[order[-1500:]].min() >= 160
+    rp, col, val, _ = oracle.build_csr(s, g, lst, 6, seed=3)
+    A = sysmat.build_csr(setup, grid, lst, 6, seed=3, staging=staging)
+    for got, want in zip(A.to_host(), (rp, col, val)):
+        np.testing.assert_array_equal(got, want)
