@@ -36,7 +36,7 @@ __global__ void k_padded_len(const int64_t* rp, int m, int64_t* plen) {
     plen[i] = (rp[i + 1] - rp[i] + 3) & ~int64_t(3);
 }
 
-__global__ void k_set_last(int64_t* p, int m, const int64_t* total) { p[m] = *total; }
+__global__ void k_set_last(int64_t* p, int64_t m, const int64_t* total) { p[m] = *total; }
 
 // One wave per row: row maximum -> scale (mixed), copy with zero padding.
 // interleave chunks: forward rows for 32 lanes x 4 entries per step, column
@@ -2387,7 +2387,7 @@ int build_groups(raptr_recon* R, const L& lists, int64_t ng, int align, int64_t*
                        lists, ng, align, cnt);
     rc = scan_exclusive_i64(cnt, *gptr, ng, tot, sws, sb, st);
     if (!rc) {
-      hipLaunchKernelGGL(k_set_last, dim3(1), dim3(1), 0, st, *gptr, int(ng),
+      hipLaunchKernelGGL(k_set_last, dim3(1), dim3(1), 0, st, *gptr, ng,
                          (const int64_t*)tot);
       (void)hipMemcpyAsync(&h, tot, 8, hipMemcpyDeviceToHost, st);
     }
@@ -3200,7 +3200,7 @@ int build_local_columns(raptr_recon* R, hipStream_t st, int rows_req = 0,
     RAPTR_HIP_TRY(pool_malloc(&tmp, 512 + sb));
     int64_t* tot = static_cast<int64_t*>(tmp);
     rc = scan_exclusive_i64(cnt, R->lup, ng, tot, static_cast<char*>(tmp) + 256, sb, st);
-    if (!rc) hipLaunchKernelGGL(k_set_last, dim3(1), dim3(1), 0, st, R->lup, int(ng),
+    if (!rc) hipLaunchKernelGGL(k_set_last, dim3(1), dim3(1), 0, st, R->lup, ng,
                                 (const int64_t*)tot);
     std::vector<int64_t> hc(static_cast<size_t>(ng));
     hipError_t le = hipGetLastError();
@@ -3601,7 +3601,8 @@ int create_plan(raptr_recon** out, int m, int n, int64_t nnz, const int64_t* d_r
         hipLaunchKernelGGL(k_padded_len, dim3(grid_for(m, 256, 8192)), dim3(256), 0, st, d_rp,
                            m, plen);
         rc = scan_exclusive_i64(plen, R->frp, m, tot, sws, sb, st);
-        if (!rc) hipLaunchKernelGGL(k_set_last, dim3(1), dim3(1), 0, st, R->frp, m, (const int64_t*)tot);
+        if (!rc) hipLaunchKernelGGL(k_set_last, dim3(1), dim3(1), 0, st, R->frp, int64_t(m),
+                                    (const int64_t*)tot);
       } else {
         (void)hipMemsetAsync(R->frp, 0, 8, st);
         (void)hipMemsetAsync(tot, 0, 8, st);
@@ -3713,7 +3714,7 @@ int create_plan(raptr_recon** out, int m, int n, int64_t nnz, const int64_t* d_r
         rc = scan_exclusive_i64(plen, R->bptr, T, tot, sws, sb, st);
       }
       if (!rc && !go) {
-        hipLaunchKernelGGL(k_set_last, dim3(1), dim3(1), 0, st, R->bptr, int(T),
+        hipLaunchKernelGGL(k_set_last, dim3(1), dim3(1), 0, st, R->bptr, T,
                            (const int64_t*)tot);
         (void)hipMemcpyAsync(&h, tot, 8, hipMemcpyDeviceToHost, st);
         hipError_t se = hipStreamSynchronize(st);
@@ -3956,7 +3957,7 @@ int raptr_recon_create_opts(raptr_recon** out, int m, int n, int64_t nnz, const 
                        d_row_order, m, plen);
     rc = scan_exclusive_i64(plen, prp, m, tot, sws, sb, st);
     if (!rc) {
-      hipLaunchKernelGGL(k_set_last, dim3(1), dim3(1), 0, st, prp, m, (const int64_t*)tot);
+      hipLaunchKernelGGL(k_set_last, dim3(1), dim3(1), 0, st, prp, int64_t(m), (const int64_t*)tot);
       hipLaunchKernelGGL(k_perm_copy, dim3(grid_for(int64_t(m) * kWave, 256, 1 << 16)),
                          dim3(256), 0, st, d_rp, d_col, d_val, d_row_order, m,
                          (const int64_t*)prp, pcol, pval);
