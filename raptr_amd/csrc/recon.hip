@@ -1285,9 +1285,9 @@ __global__ __launch_bounds__(256) void k_bwdm64(int ngc, const int64_t* __restri
 // XCDs share a range and split its bricks).  Each wave walks its brick through
 // all of its XCD's blocks; the bricks resident on one XCD at a time are
 // consecutive (neighbouring voxels) and walk the same small ratio slices
-// together, so their ratio gathers hit that XCD's L2.  Each XCD writes its
-// partial image sums to its own slice of c8; k_bwd_xreduce adds the 8
-// slices in a fixed order and applies the update.  On a device that assigns
+// together, so their ratio gathers hit that XCD's L2.  Each range's sums go
+// to its own slice of c8; k_bwd_xreduce adds the nr slices in a fixed order
+// and applies the update.  On a device that assigns
 // workgroups differently the result is the same (only the cache behaviour
 // changes).
 // boff / bcnt: this launch covers row blocks b0 + boff .. b0 + boff + bcnt
@@ -2117,9 +2117,6 @@ __global__ void k_seq_cols(int n, int64_t total, int* __restrict__ cols) {
        t += int64_t(gridDim.x) * blockDim.x)
     cols[t] = t < n ? int(t) : -1;
 }
-
-// rows of the transpose as 16-bit offsets in their row block (blocks of at
-// most 65,536 rows): 6 bytes per FP32 entry instead of 8
 
 // forward columns as 16-bit low parts (grids of <= 4 x 65,536 voxels): one
 // wave per row; split[i] packs the row's first positions with a column >=

@@ -135,10 +135,10 @@ struct raptr_recon {
   int grp_g = 16;      // members per group (16, 32)
   int* gcols = nullptr;  // ngc * grp_g member columns of the backward groups (-1: none)
   int grp_ranges = 8;  // row ranges of the kind-3 backward
-  int grp_unroll = 8;  // union entries in flight per wave (4, 8, 16)
+  int grp_unroll = 8;  // union entries per step of a forward wave (8, 16, 32)
   int grp_pipe = 1;    // kernel kind: 0 plain, 1 pipelined scalar loads, 2 matrix cores,
                        // 3 matrix cores with per-XCD row ranges in the backward
-  float* c8 = nullptr;  // kind 3: 8 partial images [8][n][64]
+  float* c8 = nullptr;  // kind 3: partial images [grp_ranges][n][64]; 1 frame: [8][n]
   int grouped_only = 0;  // no padded CSR / padded transpose (64-frame grouped passes only)
   uint16_t* brow16 = nullptr;  // transpose rows as offsets in their block (blocks <= 65,536 rows)
   int bwd_r16 = 0;             // single-frame per-XCD backward reads brow16

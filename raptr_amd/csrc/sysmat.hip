@@ -16,9 +16,9 @@
 //         (the voxel-box divisions of the slab method depend only on the
 //         plane index, so one division per plane and ray replaces six per
 //         voxel and ray, with identical float results);
-//      2. the cylinder cull runs over the grid in rounds of 1024 voxels and
-//         compacts candidates into LDS with wave ballots (ascending voxel
-//         order preserved);
+//      2. the cylinder cull takes the z intervals of 256 voxel columns at a
+//         time and compacts the voxels that pass its test into LDS with wave
+//         ballots (ascending voxel order preserved);
 //      3. candidates are sampled densely (all lanes busy), exact zeros are
 //         dropped with a second ballot compaction into an LDS row buffer;
 //      4. row buffers are flushed as pieces into a staging area and packed

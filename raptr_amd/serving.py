@@ -134,7 +134,7 @@ def estimate_lane_bytes(geometry, frames, nnz):
     g = geometry
     if frames == GROUPED_FRAMES:
         per = _GROUPED_BYTES_PER_NNZ[g.value_type] + _BUILD_BYTES_PER_NNZ
-        extra = 4 * 8 * frames * g.nvox  # per-XCD partial images
+        extra = 4 * 8 * frames * g.nvox  # partial images, at most 8
     else:
         per = _PLAN_BYTES_PER_NNZ[g.value_type] + _BUILD_BYTES_PER_NNZ
         extra = 0
