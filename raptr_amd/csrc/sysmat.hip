@@ -1487,10 +1487,11 @@ int raptr_sm_build_csr_ex(const raptr_setup_t* setup, const raptr_grid_t* grid,
     }
     total += chunk_nnz;
     first += rows;
-    // next chunk: four fifths of the staging at what these rows asked for (a
-    // count: 0.6 of it at their entries)
-    const double asked = fill ? double(hc[3]) * A.areas : double(chunk_nnz) * (0.8 / 0.6);
-    int64_t want = asked > 0 ? int64_t(0.8 * double(staging) * rows / asked) : max_rows;
+    // next chunk: 0.6 of the staging at these rows' entries, and at most 0.8 of it
+    // at what they asked for (k_sm_rays asks for a fourth to twice more than they)
+    const double per = std::max(double(chunk_nnz) / 0.6,
+                                fill ? double(hc[3]) * A.areas / 0.8 : 0.0);
+    int64_t want = per > 0 ? int64_t(double(staging) * rows / per) : max_rows;
     if (want > max_rows) want = max_rows;
     if (want < 1) want = 1;
     rows = int(want);

@@ -184,7 +184,10 @@ int make_wq_args(const raptr_setup_t* setup, const raptr_grid_t* grid, const int
   A->every = grid->n[2] < kWqFlat || entries * tiles <= kWqFewTiles;
   // (an entry has as many counters as tiles)
   const int64_t blocks = (cols + kWqBlock - 1) / kWqBlock;
-  const int64_t most = A->every || blocks > tiles ? tiles : blocks;
+  int64_t most = A->every || blocks > tiles ? tiles : blocks;
+  // a list of one workgroup a CU and more: parts of at least 4 blocks (1,718
+  // channels of 24^3 in two parts each took 168 us with their values, 157 in one)
+  if (!A->every && entries >= 256) most = blocks >= 8 ? blocks / 4 : 1;
   const int64_t want = ((A->every ? kWqFewTiles : kWqGroups) + entries - 1) / entries;
   A->parts = int(want < most ? want : most);
   A->div_yz = make_fastdiv(uint32_t(grid->n[1] * grid->n[2]));
