@@ -172,7 +172,8 @@ constexpr int64_t kWqGroups = 2048;
 // 240 x 2 cells 1,298 us, by intervals 2,176; of 240 x 240 x 4 3,083 and 2,459)
 // and on calls of at most that many tiles, which are over before the intervals
 // of the first columns stand (one channel of 96^3 51 and 70 us, of 32^3 45 and
-// 56; 64 of 32^3 59 and 57).
+// 56, 4 of 96^3 69 and 74); a fourth of them with more than 16 entries (64
+// channels of 32^3 59 and 57, 617 of 18^3, with their values, 86 and 84).
 constexpr int kWqFlat = 4;
 constexpr int64_t kWqFewTiles = 4096;
 int make_wq_args(const raptr_setup_t* setup, const raptr_grid_t* grid, const int* d_list,
@@ -181,7 +182,8 @@ int make_wq_args(const raptr_setup_t* setup, const raptr_grid_t* grid, const int
   if (entries < 1) entries = 1;
   const int64_t cols = int64_t(grid->n[0]) * grid->n[1];
   const int64_t tiles = (int64_t(A->G.nvox) + kWqTile - 1) / kWqTile;
-  A->every = grid->n[2] < kWqFlat || entries * tiles <= kWqFewTiles;
+  A->every = grid->n[2] < kWqFlat ||
+             entries * tiles <= (entries <= 16 ? kWqFewTiles : kWqFewTiles / 4);
   // (an entry has as many counters as tiles)
   const int64_t blocks = (cols + kWqBlock - 1) / kWqBlock;
   int64_t most = A->every || blocks > tiles ? tiles : blocks;
