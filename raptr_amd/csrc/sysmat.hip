@@ -1249,6 +1249,18 @@ int launch_rows(const BuildArgs& A, size_t lds, hipStream_t st, int threads = kS
       (void)hipGetLastError();
     raised.fetch_or(bit);
   }
+  // with the kernel's own arrays: a launch beyond a CU's LDS aborts the queue
+  static std::atomic<int64_t> fixed{-1};
+  int64_t own = fixed.load();
+  if (own < 0) {
+    hipFuncAttributes a;
+    RAPTR_HIP_TRY(hipFuncGetAttributes(&a, (const void*)KERNEL));
+    fixed.store(own = int64_t(a.sharedSizeBytes));
+  }
+  if (int64_t(lds) + own > 160 * 1024)
+    return fail(RAPTR_ERR_NOT_SUPPORTED,
+                "nrays=%d x planes=%d needs %lld B of LDS (> 160 KiB)", A.nrays, A.pl,
+                (long long)(int64_t(lds) + own));
   hipLaunchKernelGGL(KERNEL, dim3(unsigned(A.rows)), dim3(threads), lds, st, A);
   RAPTR_LAUNCH_CHECK();
   return RAPTR_OK;

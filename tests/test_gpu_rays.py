@@ -145,3 +145,27 @@ def test_staging_areas(gpu, oracle, staging):
     A = sysmat.build_csr(setup, grid, lst, 6, seed=3, staging=staging)
     for got, want in zip(A.to_host(), (rp, col, val)):
         np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("nz", [387, 388, 394])
+def test_candidate_build_at_the_lds_limit(gpu, oracle, nz):
+    """70 rays: the candidate build's tables with its own arrays leave a CU's 160
+    KiB from 395 planes on, the tables alone beyond 401.  It is refused there; the
+    ray masks, which need less, are not."""
+    from raptr_amd import sysmat
+    from raptr_amd import _capi as capi
+    setup, grid = two_head_setup(2, 2, 90.0), VoxelGrid((-4.0, -4.0, -97.0), (4.0, 4.0, 0.5),
+                                                        (2, 2, nz))
+    lst = np.arange(setup.nchannels, dtype=np.int32)
+    s, g = oracle_geom(oracle, setup, grid)
+    rp, col, val, _ = oracle.build_csr(s, g, lst, 70)
+    for got, want in zip(sysmat.build_csr(setup, grid, lst, 70).to_host(), (rp, col, val)):
+        np.testing.assert_array_equal(got, want)
+    if nz == 387:
+        A = sysmat.build_csr(setup, grid, lst, 70, keep_zeros=True).to_host()
+        np.testing.assert_array_equal(A[2][A[2] != 0], val)
+    else:
+        for kw in (dict(keep_zeros=True), dict(raygen=capi.RAYGEN_RAND_ELEMENT)):
+            with pytest.raises(capi.RaptrError) as e:
+                sysmat.build_csr(setup, grid, lst, 70, **kw)
+            assert e.value.status == capi.RAPTR_ERR_NOT_SUPPORTED
