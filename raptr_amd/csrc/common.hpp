@@ -46,8 +46,9 @@ inline hipStream_t S(raptr_stream_t s) { return reinterpret_cast<hipStream_t>(s)
 
 // ------------------------------------------------- device memory
 // hipMalloc and hipFree through a bounded cache of freed blocks (runtime.hip).
-// pool_free waits for the device, as hipFree does, unless the caller has
-// (pool_wait: before several of them).
+// pool_free waits for the device, as hipFree does, unless the caller has.
+// pool_wait: all work of the device has ended; unlike hipDeviceSynchronize it
+// leaves captures of other threads valid.
 hipError_t pool_malloc(void** p, size_t bytes);
 hipError_t pool_free(void* p, bool idle = false);
 hipError_t pool_wait();

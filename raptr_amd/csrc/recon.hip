@@ -4351,7 +4351,7 @@ int raptr_recon_set_fused_tiles(raptr_recon* R, int columns, int segments_per_wo
     return fail(RAPTR_ERR_INVALID_ARG, "segments per workgroup must be in 64..1048576");
   if (R->tseg && R->tshift == sh && R->tseg_target == segments_per_workgroup) return RAPTR_OK;
   clear_graphs(R);
-  (void)hipDeviceSynchronize();  // no queued pass may still read the old table
+  (void)pool_wait();  // no queued pass may still read the old table
   const int rc = build_tile_segments(R, sh, segments_per_workgroup,
                                      static_cast<hipStream_t>(stream));
   if (rc && R->fb_xcd == 2) R->fb_xcd = 1;
@@ -4369,7 +4369,7 @@ int raptr_recon_set_union_rows(raptr_recon* R, int rows, raptr_stream_t stream) 
                 "column unions need a single-frame blocked plan with a padded CSR");
   hipStream_t st = static_cast<hipStream_t>(stream);
   clear_graphs(R);
-  (void)hipDeviceSynchronize();  // no queued pass may still read the old unions
+  (void)pool_wait();  // no queued pass may still read the old unions
   rfree(R, R->lup);
   rfree(R, R->lucol);
   rfree(R, R->lcol);
@@ -4509,7 +4509,7 @@ static int mlem_impl(raptr_recon* R, int nframes, const float* d_y, float* d_x, 
       for (auto jt = R->graphs.begin(); jt != R->graphs.end(); ++jt)
         if (jt->second.used < lru->second.used) lru = jt;
       // a replay of the evicted graph may still be queued on some stream
-      RAPTR_HIP_TRY(hipDeviceSynchronize());
+      RAPTR_HIP_TRY(pool_wait());
       destroy_graph(lru->second);
       R->graphs.erase(lru);
     }

@@ -232,7 +232,7 @@ inline void destroy_graph(raptr_recon::CachedGraph& g) {
 // drained first
 inline void clear_graphs(raptr_recon* R) {
   if (R->graphs.empty()) return;
-  (void)hipDeviceSynchronize();
+  (void)pool_wait();
   for (auto& kv : R->graphs) destroy_graph(kv.second);
   R->graphs.clear();
 }

@@ -97,12 +97,17 @@ def test_frees_leave_a_capture_of_another_thread(gpu):
     def work():
         R.run(dy, dx, 1, use_graph=False, stream=st.handle)
     blocks = [DeviceArray(n, np.uint8) for n in (1 << 12, 9 << 20, 64 << 20)]
-    plans = [Reconstructor(A, sens, "f32", 1, row_order=setup)]
+    plans = [Reconstructor(A, sens, "f32", 1, row_order=setup) for _ in range(2)]
+    other = Stream()
+    dz = DeviceArray.from_numpy(np.full(A.n, 1.0 / A.n, np.float32))
+    plans[0].run(dy, dz, 5, stream=other.handle)  # a plan with captured iterations
+    other.sync()
 
     def frees():
         for b in blocks:
             b.free()
-        plans.pop().close()
+        for p in plans:
+            p.close()
         DeviceArray(9 << 20, np.uint8).free()  # a kept block, handed out and freed
     status, alone = _capture(st, work, lambda: None)
     assert status == 0 and alone >= 2
@@ -134,3 +139,41 @@ def test_cached_blocks_go_back_on_request(gpu):
     assert mem_info()[0] >= held + half
     release_cached()
     assert driver_free() >= before - half
+
+
+@pytest.mark.gpu
+def test_threads_build_run_and_free_plans(gpu):
+    """Four threads with plans and streams of their own, buffers new for every
+    run: each run captures while others allocate and free."""
+    import threading
+    import numpy as np
+    from raptr_amd import sysmat
+    from raptr_amd.device import DeviceArray, Stream
+    from raptr_amd.geometry import config_small
+    from raptr_amd.recon import Reconstructor
+    setup, grid, nrays = config_small()
+    A = sysmat.build_csr(setup, grid, np.arange(8000, dtype=np.int32), nrays)
+    sens = sysmat.sensitivity(setup, grid, nrays)
+    y = np.random.default_rng(0).poisson(5, A.m).astype(np.float32)
+    x0 = np.full(A.n, 1.0 / A.n, np.float32)
+    want = Reconstructor(A, sens, "f32", 1, row_order=setup).mlem(y, x0, 9)
+    wrong = []
+
+    def work(t):
+        try:
+            st = Stream()
+            for k in range(10):
+                R = Reconstructor(A, sens, "f32", 1, row_order=setup, stream=st.handle)
+                for _ in range(2):
+                    if not np.array_equal(R.mlem(y, x0, 9, stream=st.handle), want):
+                        wrong.append((t, k))
+                DeviceArray(5000000 + 100000 * k, np.uint8).free()
+                R.close()
+        except Exception as e:  # noqa: BLE001 - reported below
+            wrong.append((t, repr(e)))
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong, wrong[:5]
