@@ -47,8 +47,57 @@ class BlockCache {
     return (bytes + step - 1) / step * step;
   }
 
-  Error malloc(void** p, size_t bytes) {
+  // No exception leaves these (they serve C entry points): without host memory
+  // for the cache's own lists, kNoMemory.
+  Error malloc(void** p, size_t bytes) noexcept {
     *p = nullptr;
+    try {
+      return take_or_alloc(p, bytes);
+    } catch (...) {
+      if (*p) (void)d_.release(*p);
+      *p = nullptr;
+      return D::kNoMemory;
+    }
+  }
+
+  // idle: the caller has waited for the device
+  Error free(void* p, bool idle) noexcept {
+    try {
+      return keep_or_release(p, idle);
+    } catch (...) {
+      return D::kNoMemory;
+    }
+  }
+
+  // Kept blocks of a device given back to the driver, the oldest first, down to
+  // most bytes; the bytes given back.
+  size_t give_back(int dev, size_t most) noexcept {
+    try {
+      return release_kept(dev, most);
+    } catch (...) {
+      return 0;
+    }
+  }
+
+  // of the current device
+  size_t kept_bytes() {
+    int dev = 0;
+    if (d_.device(&dev) != D::kOk) return 0;
+    std::lock_guard<std::mutex> lock(mu_);
+    const auto it = kept_bytes_.find(dev);
+    return it == kept_bytes_.end() ? 0 : it->second;
+  }
+
+  D& driver() { return d_; }
+
+ private:
+  struct Block {
+    size_t bytes;
+    int dev;
+    bool kept;  // freed by its owner, in kept_
+  };
+
+  Error take_or_alloc(void** p, size_t bytes) {
     const bool ours = bytes >= kLeast && bytes <= kBlock;
     if (!ours) {
       Error e = d_.alloc(p, bytes);
@@ -77,7 +126,7 @@ class BlockCache {
     }
     size_t got = need;
     e = ours ? d_.alloc(p, need) : D::kNoMemory;
-    if (e == D::kNoMemory && give_back(dev, 0)) {
+    if (e == D::kNoMemory && release_kept(dev, 0)) {
       d_.forget_error();
       e = d_.alloc(p, need);
     }
@@ -92,8 +141,7 @@ class BlockCache {
     return e;
   }
 
-  // idle: the caller has waited for the device
-  Error free(void* p, bool idle) {
+  Error keep_or_release(void* p, bool idle) {
     if (!p) return D::kOk;
     Block b{0, 0, false};
     {
@@ -132,14 +180,12 @@ class BlockCache {
       }
       keep(p, b, false);
     }
-    (void)give_back(dev, kBytes);
+    (void)release_kept(dev, kBytes);
     return D::kOk;
   }
 
-  // Kept blocks of a device given back to the driver, the oldest first, down to
-  // most bytes; the bytes given back.  (A release can wait for the device: the
-  // lock is not held meanwhile.)
-  size_t give_back(int dev, size_t most) {
+  // (A release can wait for the device: the lock is not held meanwhile.)
+  size_t release_kept(int dev, size_t most) {
     std::list<std::pair<void*, Block>> out;
     {
       std::lock_guard<std::mutex> lock(mu_);
@@ -168,23 +214,6 @@ class BlockCache {
     }
     return bytes;
   }
-
-  // of the current device
-  size_t kept_bytes() {
-    int dev = 0;
-    if (d_.device(&dev) != D::kOk) return 0;
-    std::lock_guard<std::mutex> lock(mu_);
-    return kept_bytes_[dev];
-  }
-
-  D& driver() { return d_; }
-
- private:
-  struct Block {
-    size_t bytes;
-    int dev;
-    bool kept;  // freed by its owner, in kept_
-  };
 
   void keep(void* p, Block b, bool front) {
     b.kept = true;

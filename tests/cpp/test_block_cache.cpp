@@ -5,6 +5,7 @@
 #include <cstdio>
 #include <map>
 #include <mutex>
+#include <new>
 #include <set>
 #include <thread>
 #include <vector>
@@ -31,7 +32,7 @@ struct Model {
   uintptr_t next = 0x1000;
   size_t used = 0, room = size_t(64) << 30;
   int dev = 0, allocs = 0, releases = 0, waits = 0, clears = 0;
-  bool can_wait = true, can_release = true;
+  bool can_wait = true, can_release = true, throws = false;
   Error device(int* d) {
     *d = dev;
     return kOk;
@@ -42,6 +43,7 @@ struct Model {
     return kOk;
   }
   Error alloc(void** p, size_t bytes) {
+    if (throws) throw std::bad_alloc();
     if (used + bytes > room) return kNoMemory;
     ++allocs;
     *p = reinterpret_cast<void*>(next);
@@ -66,6 +68,7 @@ struct Model {
     return can_wait ? kOk : kNoWait;
   }
   Error clear(void* p, size_t bytes, int) {
+    if (throws) throw std::bad_alloc();
     auto it = mem.find(uintptr_t(p));
     CHECK(it != mem.end() && bytes <= it->second.bytes);  // inside the driver's block
     if (it != mem.end()) it->second.cleared = true;
@@ -204,6 +207,20 @@ static void test_give_back() {
   CHECK(c.driver().extent(other) && c.driver().mem.size() == 1);
 }
 
+// An exception below (no host memory) is an error of the call, and the lock is
+// free again.
+static void test_exceptions() {
+  Cache c;
+  void* a = get(c, 9 * MB);
+  c.driver().throws = true;
+  void* b = &c;
+  CHECK(c.malloc(&b, 30 * MB) == Model::kNoMemory && !b);
+  CHECK(c.malloc(&b, 100) == Model::kNoMemory && !b);
+  CHECK(c.free(a, false) == Model::kNoMemory);
+  c.driver().throws = false;
+  CHECK(c.free(get(c, 30 * MB), false) == Model::kOk && c.kept_bytes() >= 30 * MB);
+}
+
 // Four threads allocate, write and free blocks of a few sizes.
 static void test_threads() {
   struct Locked : Model {
@@ -250,6 +267,7 @@ int main() {
   test_bounds();
   test_no_wait();
   test_give_back();
+  test_exceptions();
   test_threads();
   std::printf("%d failure(s)\n", failures);
   return failures != 0;
